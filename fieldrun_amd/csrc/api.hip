@@ -443,8 +443,8 @@ frq_w* frq_upload_i4(frq_ctx* c, const uint8_t* packed,
     Weight& w = h->w;
     w.dtype = FRQ_DT_I4; w.device = c->device; w.n = n; w.k = k; w.g = g;
     const size_t rb = (k + 1) / 2, ng = (k + g - 1) / g;
-    hipError_t e = hipMalloc(&w.q4raw, n * rb + 16);
-    if (e == hipSuccess) e = hipMalloc(&w.s4raw, n * ng * 2 + 16);
+    hipError_t e = hipMalloc(&w.q4raw, n * rb + FRQ_PACK_PAD);
+    if (e == hipSuccess) e = hipMalloc(&w.s4raw, n * ng * 2 + FRQ_PACK_PAD);
     if (e == hipSuccess && n * rb)
         e = hipMemcpyAsync(w.q4raw, packed, n * rb, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess && n * ng)
@@ -481,8 +481,8 @@ frq_w* frq_upload_q4a(frq_ctx* c, const uint8_t* packed, const uint16_t* scale_f
     w.rpitch = q4a_pitch(k);
     std::vector<uint32_t> sm(n * ng);
     for (size_t i = 0; i < n * ng; ++i) sm[i] = (uint32_t)scale_f16[i] | ((uint32_t)min_f16[i] << 16);
-    hipError_t e = hipMalloc(&w.q4raw, n * w.rpitch + 16);
-    if (e == hipSuccess) e = hipMalloc(&w.q4a_sm, n * ng * 4 + 16);
+    hipError_t e = hipMalloc(&w.q4raw, n * w.rpitch + FRQ_PACK_PAD);
+    if (e == hipSuccess) e = hipMalloc(&w.q4a_sm, n * ng * 4 + FRQ_PACK_PAD);
     if (e == hipSuccess) e = hipMemsetAsync(w.q4raw, 0, n * w.rpitch + 16, c->stream);
     if (e == hipSuccess && n * rb)
         e = hipMemcpy2DAsync(w.q4raw, w.rpitch, packed, rb, rb, n, hipMemcpyHostToDevice, c->stream);
@@ -924,9 +924,9 @@ static frq_moe_w* moe_upload_ex(frq_ctx* c, int dtype, size_t n_exp, size_t d, s
         m.out = out;
         const size_t ng = q ? (in + g - 1) / g : 0;
         const size_t per = q ? out * ((in + 1) / 2) : in * out * (dtype == FRQ_DT_F16 ? 2 : 4);
-        e = hipMalloc(&m.raw, n_exp * per);
-        if (e == hipSuccess && q) e = hipMalloc(&m.sc, n_exp * out * ng * 2);
-        if (e == hipSuccess && dtype == FRQ_DT_Q4A) e = hipMalloc(&m.mn, n_exp * out * ng * 2);
+        e = hipMalloc(&m.raw, n_exp * per + FRQ_PACK_PAD);
+        if (e == hipSuccess && q) e = hipMalloc(&m.sc, n_exp * out * ng * 2 + FRQ_PACK_PAD);
+        if (e == hipSuccess && dtype == FRQ_DT_Q4A) e = hipMalloc(&m.mn, n_exp * out * ng * 2 + FRQ_PACK_PAD);
         for (size_t x = 0; x < n_exp && e == hipSuccess; ++x) {
             if (!raw[x] || (q && !sc[x]) || (dtype == FRQ_DT_Q4A && !mn[x])) {
                 e = hipErrorInvalidValue;

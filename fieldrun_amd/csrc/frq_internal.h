@@ -33,6 +33,7 @@
 #define FRQ_T 32            // OUTLIER_T (src/bundle.rs:309)
 #define FRQ_KALIGN 128      // Kp alignment (a multiple of the GEMM k-step)
 #define FRQ_NALIGN 256      // Np alignment (a multiple of every N tile)
+#define FRQ_PACK_PAD 64      // bytes readable past packed int4 rows and their scales (mm_f32.hip)
 #define FRQ_MALIGN 128      // Mp alignment of the a8 workspace (GEMM M tile)
 
 namespace frq {
@@ -556,6 +557,30 @@ size_t i4_blocked_bytes(size_t n, size_t k);
 hipError_t launch_i4_block(const uint8_t* raw, const uint16_t* sraw, size_t n,
                            size_t k, uint8_t* blk, uint16_t* sblk,
                            hipStream_t s);
+// A weight in its stored bytes, for launch_mm_f32.  Packed (i4, q4a): rows of
+// ceil(k / 2) bytes at a pitch, even k in the low nibble, f16 scales (q4a:
+// and mins) of n rows x ng groups, ss apart; FRQ_PACK_PAD bytes past the last
+// row and the last scale are readable.  f16 / f32: (k, n) row-major.  per / sper: weight elements
+// (packed: bytes) and scales of one expert.
+struct MmWeight {
+    const void* w;
+    const uint16_t *sc, *mn;
+    int ss, n, k, g, ng;
+    size_t pitch, per, sper;
+};
+// A grouped product's rows: tile t holds up to `rows` (<= MM_GROUP_ROWS) rows
+// of expert tile_e[t] from its row tile_r[t], of rows off[e] .. off[e] + cnt[e] of the
+// permutation; the activation row is ptok[row] (gather) or the row itself.
+struct MmGroup {
+    const int32_t *ptok, *off, *cnt, *tile_e, *tile_r, *ntile;
+    int gather, rows;
+};
+constexpr int MM_GROUP_ROWS = 32;
+// a (m, k) f32 times the weight (dt FRQ_DT_I4 / Q4A / F16 / F32) in a.dot's
+// order, any m, k, n and group; the grouped form over at most ntile tiles.
+hipError_t launch_mm_f32(int dt, const MmWeight& w, const float* a, size_t m, float* out, int cus, hipStream_t s);
+hipError_t launch_mm_f32_group(int dt, const MmWeight& w, const MmGroup& grp, unsigned ntile, const float* a,
+                               float* out, int cus, hipStream_t s);
 // Affine int4 (q4a) linear (any m): packed rows in q4raw at pitch rpitch.
 size_t q4a_pitch(size_t k);
 hipError_t launch_q4a(const Weight& w, size_t m, const float* a, float* out, hipStream_t s);

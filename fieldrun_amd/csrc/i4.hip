@@ -32,8 +32,7 @@
 // workgroups would need device-scope fences, which on this part write back
 // and invalidate the whole L2.
 // Other shapes run i4_gemv_generic (M == 1, bit-identical to i4_dot_avx2)
-// or, M > 1 in the exact order, i4_mm_dpp (K % 32 == 0, g % 16 == 0),
-// i4_rows_chain (K and g multiples of 32) or i4_gemm_rows.  Up to 16
+// or, M > 1 in the exact order, the f32 matrix cores (mm_f32.hip).  Up to 16
 // independent M == 1 rows (a batched decode) run i4_rows_dpp.
 #include "frq_internal.h"
 
@@ -315,151 +314,6 @@ __device__ __forceinline__ void dpp_fma16(float (&l)[8], float w, const float (&
 #undef FRQ_DPP_C0
 #undef FRQ_DPPF
 
-// One k of R FMA chains: c[r] = fma(w_r(lane n), a, c[r]) for r < R, where
-// v_fmac_f32_dpp row_newbcast:n gives every token lane of a 16-lane DPP row
-// the weight held by lane n of that row (lane n: k0 + n).  The s_nop gives
-// the two wait states a DPP read needs after the VALU write of the weights.
-#define FRQ_CHF(acc, w, a, n) "v_fmac_f32_dpp %" #acc ", %" #w ", %" #a " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
-#define FRQ_CH8(n)                                                                                       \
-    FRQ_CHF(0, 8, 16, n) FRQ_CHF(1, 9, 16, n) FRQ_CHF(2, 10, 16, n) FRQ_CHF(3, 11, 16, n) FRQ_CHF(4, 12, 16, n) \
-    FRQ_CHF(5, 13, 16, n) FRQ_CHF(6, 14, 16, n) FRQ_CHF(7, 15, 16, n)
-#define FRQ_CH8_OPS                                                                                          \
-    : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]), "+v"(c[7])         \
-    : "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(a)
-#define FRQ_CH8_CASE(n) \
-    if constexpr (N == n) asm("s_nop 1\n\t" FRQ_CH8(n) FRQ_CH8_OPS);
-template <int N>
-__device__ __forceinline__ void dpp_chain8(float (&c)[8], const float (&w)[8], float a) {
-    FRQ_CH8_CASE(0) FRQ_CH8_CASE(1) FRQ_CH8_CASE(2) FRQ_CH8_CASE(3) FRQ_CH8_CASE(4) FRQ_CH8_CASE(5)
-    FRQ_CH8_CASE(6) FRQ_CH8_CASE(7) FRQ_CH8_CASE(8) FRQ_CH8_CASE(9) FRQ_CH8_CASE(10) FRQ_CH8_CASE(11)
-    FRQ_CH8_CASE(12) FRQ_CH8_CASE(13) FRQ_CH8_CASE(14) FRQ_CH8_CASE(15)
-}
-#undef FRQ_CH8_CASE
-#undef FRQ_CH8_OPS
-#undef FRQ_CH8
-#undef FRQ_CHF
-
-// M > 1 rows in a.dot's order (each output: MM_KC-long k blocks, each an
-// FMA chain from +0 over k with w = s4 * scale, the blocks added in order)
-// with the weights broadcast across tokens: lane 16 d + t of a wave is
-// token t of the workgroup's 16-row tile (blockIdx.y) in DPP row d.  The
-// ND = 4 NW DPP rows D = BP rs + ph form ND / BP row sets of BP block
-// phases: row set rs owns the R weight rows r0 + R rs .. + R - 1, phase ph
-// takes blocks ph, ph + BP, ... .  For each 16-k chunk a lane dequantises
-// its rows' 16 weights into one register a row (lane n: k0 + n, exact
-// s4 * scale) and dpp_chain8 advances the R chains one k at a time; the
-// chunk's activations are the lane's own 16 (row-major), one chunk ahead.
-// A block's chain values go to LDS; after a slice of BP blocks, one barrier,
-// and the lane of each (row, token) adds them to its running sum in block
-// order (blocks past the end add +0, which a sum from +0 absorbs: no chain
-// from +0 ends at -0).  Needs K % 32 == 0, g % 16 == 0, M rows of K floats
-// 16-byte aligned.
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void i4_mm_dpp(const uint8_t* __restrict__ packed,
-                                                     const uint16_t* __restrict__ scale, int N, int K, int g,
-                                                     const float* __restrict__ a, int M, float* __restrict__ out,
-                                                     int BP) {
-    constexpr int R = 8, ND = 4 * NW;
-    constexpr int TB = ND * R * 16 * 2;  // term floats a buffer (RS R 16 pairs, BP + 1 apart)
-    __shared__ float tb[2][TB];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int t = lane & 15, D = 4 * wave + (lane >> 4);
-    const int RS = ND / BP, rs = D / BP, ph = D - rs * BP, TS = BP + 1;
-    const int nb = (K + MM_KC - 1) / MM_KC, nsl = (nb + BP - 1) / BP;
-    const int rows = RS * R, r0 = blockIdx.x * rows + rs * R, m0 = blockIdx.y * 16;
-    const int ng = (K + g - 1) / g;
-    const size_t pitch = (size_t)K / 2;
-    const uint8_t* wrow[R];
-    const uint16_t* srow[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const size_t row = (size_t)min(r0 + r, N - 1);  // clamped: loads stay unconditional
-        wrow[r] = packed + row * pitch + 4 * (t >> 3);
-        srow[r] = scale + row * ng;
-    }
-    const float* ar = a + (size_t)min(m0 + t, M - 1) * K;
-    const int sh = 4 * (t & 7);
-    // this lane's chunk sequence: slice s, chunk q of block s BP + ph
-    // (clamped to the last chunk of the row past the end: its values go
-    // unused)
-    const int nck = (K / 16);
-    auto chunk_k = [&](int s, int q) { return min((s * BP + ph) * MM_KC + 16 * q, 16 * (nck - 1)); };
-    struct Ld {
-        uint32_t w[R];
-        uint32_t sc[R];
-        float4 a[4];
-    };
-    auto load = [&](int k0, Ld& b) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) b.w[r] = *reinterpret_cast<const uint32_t*>(wrow[r] + (uint32_t)k0 / 2);
-        const uint32_t so = 2 * (uint32_t)(k0 / g);
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            b.sc[r] = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(srow[r]) + so);
-        const float4* ap = reinterpret_cast<const float4*>(ar + k0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) b.a[i] = ap[i];
-    };
-    auto issued = [] {
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    float c[R];
-    auto chunk = [&](const Ld& b) {
-        float wv[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            wv[r] = (float)(int)__builtin_amdgcn_sbfe((int)b.w[r], sh, 4) * h2f((uint16_t)b.sc[r]);
-        const float av[16] = {b.a[0].x, b.a[0].y, b.a[0].z, b.a[0].w, b.a[1].x, b.a[1].y, b.a[1].z, b.a[1].w,
-                              b.a[2].x, b.a[2].y, b.a[2].z, b.a[2].w, b.a[3].x, b.a[3].y, b.a[3].z, b.a[3].w};
-        dpp_chain8<0>(c, wv, av[0]); dpp_chain8<1>(c, wv, av[1]); dpp_chain8<2>(c, wv, av[2]);
-        dpp_chain8<3>(c, wv, av[3]); dpp_chain8<4>(c, wv, av[4]); dpp_chain8<5>(c, wv, av[5]);
-        dpp_chain8<6>(c, wv, av[6]); dpp_chain8<7>(c, wv, av[7]); dpp_chain8<8>(c, wv, av[8]);
-        dpp_chain8<9>(c, wv, av[9]); dpp_chain8<10>(c, wv, av[10]); dpp_chain8<11>(c, wv, av[11]);
-        dpp_chain8<12>(c, wv, av[12]); dpp_chain8<13>(c, wv, av[13]); dpp_chain8<14>(c, wv, av[14]);
-        dpp_chain8<15>(c, wv, av[15]);
-    };
-    const int P = rows * 16;  // (row, token) pairs: pair p = (row p / 16, token p % 16)
-    float sum[(ND * R * 16 + 64 * NW - 1) / (64 * NW)];
-    constexpr int PPT = (ND * R * 16 + 64 * NW - 1) / (64 * NW);  // pairs a thread at most
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) sum[i] = 0.0f;
-    Ld b0, b1;
-    load(chunk_k(0, 0), b0);
-    for (int s = 0; s < nsl; ++s) {
-        const int blk = s * BP + ph;
-        const int nq = blk < nb ? min(16, (K - blk * MM_KC) / 16) : 16;  // past the end: any 16, unused
-#pragma unroll
-        for (int r = 0; r < R; ++r) c[r] = 0.0f;
-        // chunks in pairs (K % 32 == 0: every block has an even count); the
-        // last pair's second load is the next slice's first chunk
-        for (int q = 0; q < nq; q += 2) {
-            load(chunk_k(s, q + 1), b1);
-            issued();
-            chunk(b0);
-            load(q + 2 < nq ? chunk_k(s, q + 2) : chunk_k(s + 1, 0), b0);
-            issued();
-            chunk(b1);
-        }
-        float* tbs = tb[s & 1];
-#pragma unroll
-        for (int r = 0; r < R; ++r) tbs[((rs * R + r) * 16 + t) * TS + ph] = blk < nb ? c[r] : 0.0f;
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < PPT; ++i) {
-            const int p = tid + 64 * NW * i;
-            if (p < P)
-                for (int j = 0; j < BP; ++j) sum[i] = sum[i] + tbs[p * TS + j];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-        const int p = tid + 64 * NW * i;
-        const int row = blockIdx.x * rows + p / 16, tok = m0 + p % 16;
-        if (p < P && row < N && tok < M) out[(size_t)tok * N + row] = sum[i];
-    }
-}
-
 // The activation layout of i4_rows_dpp: the 16 token rows interleaved by
 // k-quads, a4[64 (k / 4) + 4 t + k % 4] = a[t][k] (rows t >= M zero), so
 // that the 16 token lanes of a DPP row read 256 contiguous bytes a load.
@@ -620,112 +474,6 @@ __global__ __launch_bounds__(64 * NW) void i4_rows_dpp(const uint8_t* __restrict
         const int pr = p >> 4, pt = p & 15;
         if (pt < M && r0 + pr < N) out[(size_t)pt * N + r0 + pr] = sum;
     }
-}
-
-// M > 1: dequantise w = s4 * scale (f32, exact) and sum in a.dot's order
-// (MM_KC-long k blocks, each an FMA chain from +0, added in order).  One
-// thread per column j and
-// up to 16 token rows; the token rows' activations are uniform across the
-// wave (scalar loads), the weight row is the thread's own packed row.
-template <int MT>
-__global__ __launch_bounds__(256) void i4_gemm_rows(
-    const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scale,
-    int N, int K, int g, const float* __restrict__ a, int M,
-    float* __restrict__ out) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int m0 = blockIdx.y * MT;
-    if (j >= N) return;
-    const int rb = (K + 1) / 2, ng = (K + g - 1) / g;
-    const uint8_t* prow = packed + (size_t)j * rb;
-    const uint16_t* srow = scale + (size_t)j * ng;
-    float acc[MT], tot[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) tot[m] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += MM_KC) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = 0.0f;
-        for (int kk = k0; kk < min(K, k0 + MM_KC); ++kk) {
-            const uint8_t byte = prow[kk >> 1];
-            const int v = (kk & 1) ? (byte >> 4) : (byte & 0x0F);
-            const float w = (float)((int)((uint32_t)v << 28) >> 28) * h2f(srow[kk / g]);
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                if (m0 + m < M) acc[m] = __builtin_fmaf(a[(size_t)(m0 + m) * K + kk], w, acc[m]);
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m) tot[m] = tot[m] + acc[m];
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-        if (m0 + m < M) out[(size_t)(m0 + m) * N + j] = tot[m];
-}
-
-// The same chain with one thread per (column j, token row blockIdx.y), for
-// K % 32 == 0, g % 32 == 0 and 16-byte aligned activation rows: the thread
-// reads its packed row 32 nibbles (16 bytes) at a time and the token's 32
-// activations (uniform across the workgroup) with them, one chunk ahead of
-// the chain, so the FMA chain is the only serial part.  The order per output
-// is i4_gemm_rows' (a.dot's blocks over kk, w = s4 * scale), bit for bit.
-__global__ __launch_bounds__(256) void i4_rows_chain(const uint8_t* __restrict__ packed,
-                                                     const uint16_t* __restrict__ scale, int N, int K, int g,
-                                                     const float* __restrict__ a, float* __restrict__ out) {
-    const int j = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
-    const int jj = min(j, N - 1);  // clamped: the loads stay unconditional, the store is guarded
-    const int nc = K / 32, ng = K / g;
-    const uint4* prow = reinterpret_cast<const uint4*>(packed + (size_t)jj * (K / 2));
-    const uint16_t* srow = scale + (size_t)jj * ng;
-    const float4* arow = reinterpret_cast<const float4*>(a + (size_t)m * K);
-    struct Chunk {
-        uint4 w;
-        float s;
-        float4 av[8];
-    };
-    auto ld = [&](Chunk& c, int i) {
-        c.w = prow[i];
-        c.s = h2f(srow[(32 * i) / g]);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) c.av[u] = arow[8 * i + u];
-    };
-    float acc = 0.0f;
-    auto chain = [&](const Chunk& c) {
-        const uint32_t ws[4] = {c.w.x, c.w.y, c.w.z, c.w.w};
-#pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4) {
-            const float x[8] = {c.av[2 * c4].x, c.av[2 * c4].y, c.av[2 * c4].z, c.av[2 * c4].w,
-                                c.av[2 * c4 + 1].x, c.av[2 * c4 + 1].y, c.av[2 * c4 + 1].z, c.av[2 * c4 + 1].w};
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc = __builtin_fmaf(x[q], s4f(ws[c4], q) * c.s, acc);
-        }
-    };
-    // a.dot's blocks: MM_KC / 32 chunks (an even count) each, so a block
-    // starts on an even chunk, where the running block sum is folded in
-    static_assert(MM_KC % 64 == 0, "blocks start on even chunks");
-    float tot = 0.0f;
-    auto fold = [&](int i) {
-        if (i > 0 && i % (MM_KC / 32) == 0) {
-            tot = tot + acc;
-            acc = 0.0f;
-        }
-    };
-    Chunk c0, c1;
-    ld(c0, 0);
-    ld(c1, min(1, nc - 1));
-    __builtin_amdgcn_sched_barrier(0);
-    int i = 0;
-    for (; i + 2 <= nc; i += 2) {
-        fold(i);
-        chain(c0);
-        ld(c0, min(i + 2, nc - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        chain(c1);
-        ld(c1, min(i + 3, nc - 1));
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (i < nc) {
-        fold(i);
-        chain(c0);
-    }
-    if (j < N) out[(size_t)m * N + j] = tot + acc;
 }
 
 constexpr float XMAX4 = 8323072.0f;  // 127 * 2^16
@@ -1407,6 +1155,23 @@ hipError_t launch_i4_m1_rows(const Weight& w, size_t m, const float* a, float* o
     return hipSuccess;
 }
 
+namespace {
+// M > 1: the dequantised weights on the f32 matrix cores, in a.dot's order.
+hipError_t mm_dequant(const Weight& w, size_t m, const float* a, float* out, hipStream_t s) {
+    if (w.n > (size_t)INT32_MAX || w.k > (size_t)INT32_MAX) return hipErrorInvalidValue;
+    MmWeight v{};
+    v.w = w.q4raw;
+    v.sc = w.s4raw;
+    v.ss = 1;
+    v.n = (int)w.n;
+    v.k = (int)w.k;
+    v.g = (int)std::min(w.g, std::max<size_t>(w.k, 1));  // a longer group is one group
+    v.ng = (int)((w.k + w.g - 1) / w.g);
+    v.pitch = (w.k + 1) / 2;
+    return launch_mm_f32(FRQ_DT_I4, v, a, m, out, device_cus(w.device), s);
+}
+}  // namespace
+
 hipError_t launch_i4_exact(const Weight& w, size_t m, const float* a, float* out, hipStream_t s) {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (m == 1) {
@@ -1416,42 +1181,7 @@ hipError_t launch_i4_exact(const Weight& w, size_t m, const float* a, float* out
             w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, out);
         return hipGetLastError();
     }
-    if (w.k % 32 == 0 && w.g % 16 == 0 && ((uintptr_t)a & 15) == 0 && (m + 15) / 16 <= 65535 &&
-        w.k <= (size_t)INT32_MAX && w.n <= (size_t)INT32_MAX && w.n * w.k / 2 < ((size_t)1 << 32)) {
-        // workgroups of NW waves (4 NW DPP rows) in BP block phases: the
-        // most blocks used of the slices run, then the longer slice (fewer
-        // rows a workgroup, fewer barriers), then four waves
-        const int nb = (int)((w.k + MM_KC - 1) / MM_KC);
-        int bnw = 4, bbp = 1;
-        double best = -1.0;
-        for (int nw : {4, 3})
-            for (int bp = 1; bp <= 4 * nw; ++bp) {
-                if ((4 * nw) % bp) continue;
-                const double eff = (double)nb / ((nb + bp - 1) / bp * bp);
-                if (eff > best + 1e-9 || (eff > best - 1e-9 && bp > bbp)) {
-                    best = eff;
-                    bnw = nw;
-                    bbp = bp;
-                }
-            }
-        const unsigned rows = (unsigned)(4 * bnw / bbp * 8);
-        const dim3 grid((unsigned)((w.n + rows - 1) / rows), (unsigned)((m + 15) / 16));
-        if (bnw == 3)
-            i4_mm_dpp<3><<<grid, dim3(192), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, (int)m, out,
-                                                    bbp);
-        else
-            i4_mm_dpp<4><<<grid, dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, (int)m, out,
-                                                    bbp);
-        return hipGetLastError();
-    }
-    if (w.k % 32 == 0 && w.g % 32 == 0 && ((uintptr_t)a & 15) == 0 && m <= 65535) {
-        i4_rows_chain<<<dim3((unsigned)((w.n + 255) / 256), (unsigned)m), dim3(256), 0, s>>>(
-            w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, out);
-        return hipGetLastError();
-    }
-    dim3 grid((unsigned)((w.n + 255) / 256), (unsigned)((m + 15) / 16));
-    i4_gemm_rows<16><<<grid, dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, (int)m, out);
-    return hipGetLastError();
+    return mm_dequant(w, m, a, out, s);
 }
 
 hipError_t launch_i4(const Weight& w, size_t m, const float* a, float* out,
@@ -1483,10 +1213,7 @@ hipError_t launch_i4(const Weight& w, size_t m, const float* a, float* out,
             w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, out);
         return hipGetLastError();
     }
-    dim3 grid((unsigned)((w.n + 255) / 256), (unsigned)((m + 15) / 16));
-    i4_gemm_rows<16><<<grid, dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k,
-                                                (int)w.g, a, (int)m, out);
-    return hipGetLastError();
+    return mm_dequant(w, m, a, out, s);
 }
 
 }  // namespace frq

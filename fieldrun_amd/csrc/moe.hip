@@ -1367,75 +1367,21 @@ __device__ float exact_ex(const float* __restrict__ x, const ExpView& v, size_t 
     return c;
 }
 
-// expert_mm of one expert: a thread per (row, output column).
-template <int DT>
-__global__ __launch_bounds__(256) void expert_mm_ex_kernel(const float* __restrict__ x, int m, ExpView v, int e,
-                                                           float* __restrict__ y) {
-    const int j = blockIdx.x * 256 + threadIdx.x, i = blockIdx.y;
-    if (j >= v.out || i >= m) return;
-    y[(size_t)i * v.out + j] = exact_ex<DT>(x + (size_t)i * v.in, v, (size_t)e, j);
-}
-
-// Grouped expert matmul over the tile list in expert_mm's own order, for any
-// stored dtype: workgroup (tile of up to GM_TR rows of one expert, 64
-// output columns); a lane per column, wave w the tile's rows w, w + 4, ...;
-// the tile's x rows pass through LDS one a.dot block at a time, each weight
-// value formed once for all of the wave's rows.  src = ptok[prow] when gather
-// (rows of x), else prow.
-constexpr int EX_RW = GM_TR / 4;  // rows a wave
-
-template <int DT>
-__global__ __launch_bounds__(256) void moe_ex_kernel(ExpView v, const float* __restrict__ x, int gather,
-                                                     const int32_t* __restrict__ ptok,
-                                                     const int32_t* __restrict__ off,
-                                                     const int32_t* __restrict__ cnt,
-                                                     const int32_t* __restrict__ tile_e,
-                                                     const int32_t* __restrict__ tile_r,
-                                                     const int32_t* __restrict__ ntile, float* __restrict__ y) {
-    __shared__ float xs[GM_TR][MM_KC + 1];
-    __shared__ int srcs[GM_TR];
-    const int tix = blockIdx.x;
-    if (tix >= ntile[0]) return;  // uniform
-    const int e = tile_e[tix], r0 = tile_r[tix];
-    const int rows = min(GM_TR, cnt[e] - r0), pbase = off[e] + r0;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid < GM_TR) {
-        const int prow = pbase + min(tid, rows - 1);
-        srcs[tid] = gather ? ptok[prow] : prow;
-    }
-    const int j = blockIdx.y * 64 + lane, jc = min(j, v.out - 1);
-    const int K = v.in;
-    float tot[EX_RW], acc[EX_RW];
-#pragma unroll
-    for (int u = 0; u < EX_RW; ++u) tot[u] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += MM_KC) {
-        const int kn = min(MM_KC, K - k0);
-        __syncthreads();  // srcs written / the previous block's xs read
-        for (int idx = tid; idx < rows * kn; idx += 256) {
-            const int r = idx / kn, kk = idx - r * kn;
-            xs[r][kk] = x[(size_t)srcs[r] * K + k0 + kk];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < EX_RW; ++u) acc[u] = 0.0f;
-        for (int kk = 0; kk < kn; ++kk) {
-            const float w = wval<DT>(v, (size_t)e, k0 + kk, jc);
-#pragma unroll
-            for (int u = 0; u < EX_RW; ++u) {
-                const int r = wave + 4 * u;
-                if (r < rows) acc[u] = __builtin_fmaf(xs[r][kk], w, acc[u]);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < EX_RW; ++u) tot[u] = tot[u] + acc[u];
-    }
-    if (j < v.out) {
-#pragma unroll
-        for (int u = 0; u < EX_RW; ++u) {
-            const int r = wave + 4 * u;
-            if (r < rows) y[(size_t)(pbase + r) * v.out + j] = tot[u];
-        }
-    }
+// The matrix as launch_mm_f32 takes it.
+MmWeight mm_weight(const ExpView& v) {
+    MmWeight w{};
+    w.w = v.raw;
+    w.sc = v.sc;
+    w.mn = v.mn;
+    w.ss = 1;
+    w.n = v.out;
+    w.k = v.in;
+    w.g = std::min(v.g, std::max(v.in, 1));
+    w.ng = v.ng;
+    w.pitch = (size_t)v.rb;
+    w.per = v.per;
+    w.sper = v.sper;
+    return w;
 }
 
 // ---- int4 experts on the int8 MFMA ------------------------------------------
@@ -2008,8 +1954,9 @@ static hipError_t moe_gmm_pair(unsigned nt, const GmmArgs& g0, const GmmArgs& g1
 }
 
 // One grouped matmul of a non-int8 bank matrix: the int4 MFMA kernel where
-// the bank has the operand copy (g % 32 == 0), else expert_mm's own order.
-static hipError_t moe_ex_mm(const MoeBank& b, const ExpMat& m, unsigned nt, int gather, const int8_t* D,
+// the bank has the operand copy (g % 32 == 0), else expert_mm's own order on
+// the f32 matrix cores (mm_f32.hip).
+static hipError_t moe_ex_mm(const MoeBank& b, const ExpMat& m, unsigned nt, size_t tr, int gather, const int8_t* D,
                             const float* dso, size_t kp, const float* xf, const MoeWs& ws, float* y,
                             const ExpMat* m2, float* y2, hipStream_t s) {
     const ExpView v = exp_view(b, m);
@@ -2028,27 +1975,9 @@ static hipError_t moe_ex_mm(const MoeBank& b, const ExpMat& m, unsigned nt, int 
             a, a2, ncg1, gather, ws.ptok, ws.off, ws.cnt, ws.tile_e, ws.tile_r, ws.ntile);
         return hipGetLastError();
     }
-    const dim3 grid(nt, (unsigned)((m.out + 63) / 64));
-    switch (b.dtype) {
-        case FRQ_DT_I4:
-            moe_ex_kernel<FRQ_DT_I4><<<grid, dim3(256), 0, s>>>(v, xf, gather, ws.ptok, ws.off, ws.cnt, ws.tile_e,
-                                                                ws.tile_r, ws.ntile, y);
-            break;
-        case FRQ_DT_Q4A:
-            moe_ex_kernel<FRQ_DT_Q4A><<<grid, dim3(256), 0, s>>>(v, xf, gather, ws.ptok, ws.off, ws.cnt, ws.tile_e,
-                                                                 ws.tile_r, ws.ntile, y);
-            break;
-        case FRQ_DT_F16:
-            moe_ex_kernel<FRQ_DT_F16><<<grid, dim3(256), 0, s>>>(v, xf, gather, ws.ptok, ws.off, ws.cnt, ws.tile_e,
-                                                                 ws.tile_r, ws.ntile, y);
-            break;
-        default:
-            moe_ex_kernel<FRQ_DT_F32><<<grid, dim3(256), 0, s>>>(v, xf, gather, ws.ptok, ws.off, ws.cnt, ws.tile_e,
-                                                                 ws.tile_r, ws.ntile, y);
-            break;
-    }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && m2) return moe_ex_mm(b, *m2, nt, gather, D, dso, kp, xf, ws, y2, nullptr, nullptr, s);
+    const MmGroup grp{ws.ptok, ws.off, ws.cnt, ws.tile_e, ws.tile_r, ws.ntile, gather, (int)tr};
+    const hipError_t e = launch_mm_f32_group(b.dtype, mm_weight(v), grp, nt, xf, y, device_cus(b.device), s);
+    if (e == hipSuccess && m2) return moe_ex_mm(b, *m2, nt, tr, gather, D, dso, kp, xf, ws, y2, nullptr, nullptr, s);
     return e;
 }
 
@@ -2095,13 +2024,13 @@ static hipError_t launch_moe_ex(const MoeBank& b, const float* x, size_t T, cons
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     const bool silu_ = b.act == FRQ_ACT_SILU;
-    if ((e = moe_ex_mm(b, b.mg, nt, 1, ws.xd, ws.xso, b.kpd, x, ws, ws.g, silu_ ? &b.mu : nullptr, ws.u, s)) !=
+    if ((e = moe_ex_mm(b, b.mg, nt, tr, 1, ws.xd, ws.xso, b.kpd, x, ws, ws.g, silu_ ? &b.mu : nullptr, ws.u, s)) !=
         hipSuccess)
         return e;
     act_digits_kernel<<<dim3((unsigned)(T * topk)), dim3(256), 0, s>>>(
         ws.g, ws.u, b.act, mi, gw, (int)b.kpm, ws.off, E, ws.h, ws.hd, ws.hso);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = moe_ex_mm(b, b.md, nt, 0, ws.hd, ws.hso, b.kpm, ws.h, ws, ws.dn, nullptr, nullptr, s)) != hipSuccess)
+    if ((e = moe_ex_mm(b, b.md, nt, tr, 0, ws.hd, ws.hso, b.kpm, ws.h, ws, ws.dn, nullptr, nullptr, s)) != hipSuccess)
         return e;
     combine_kernel<<<dim3((unsigned)(((d % 4 ? d : d / 4) + 255) / 256), (unsigned)T), dim3(256), 0, s>>>(
         ws.dn, ws.sel, ws.w, ws.pos, (int)topk, d, out);
@@ -2111,16 +2040,12 @@ static hipError_t launch_moe_ex(const MoeBank& b, const float* x, size_t T, cons
 hipError_t launch_expert_mm_ex(const MoeBank& b, const ExpMat& mt, size_t e, const float* x, size_t m, float* y,
                                hipStream_t st) {
     if (m == 0) return hipSuccess;
-    const ExpView v = exp_view(b, mt);
-    const dim3 grid((unsigned)((mt.out + 255) / 256), (unsigned)m);
-    switch (b.dtype) {
-        case FRQ_DT_I4: expert_mm_ex_kernel<FRQ_DT_I4><<<grid, dim3(256), 0, st>>>(x, (int)m, v, (int)e, y); break;
-        case FRQ_DT_Q4A: expert_mm_ex_kernel<FRQ_DT_Q4A><<<grid, dim3(256), 0, st>>>(x, (int)m, v, (int)e, y); break;
-        case FRQ_DT_F16: expert_mm_ex_kernel<FRQ_DT_F16><<<grid, dim3(256), 0, st>>>(x, (int)m, v, (int)e, y); break;
-        case FRQ_DT_F32: expert_mm_ex_kernel<FRQ_DT_F32><<<grid, dim3(256), 0, st>>>(x, (int)m, v, (int)e, y); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    MmWeight w = mm_weight(exp_view(b, mt));
+    const bool q = b.dtype == FRQ_DT_I4 || b.dtype == FRQ_DT_Q4A;
+    w.w = (const char*)w.w + e * w.per * (q ? 1 : b.dtype == FRQ_DT_F16 ? 2 : 4);
+    if (w.sc) w.sc += e * w.sper;
+    if (w.mn) w.mn += e * w.sper;
+    return launch_mm_f32(b.dtype, w, x, m, y, device_cus(b.device), st);
 }
 
 hipError_t launch_moe_i4_block(ExpMat& mt, size_t E, size_t g, hipStream_t st) {

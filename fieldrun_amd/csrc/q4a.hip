@@ -11,9 +11,8 @@
 //           sum += scale*qsum + min*asum across the groups in order.
 //   M > 1:  the dequantised weight (scale*q + min, a mul then an add) and
 //           a.dot's order per output (matrixmultiply's sgemm: MM_KC-long k
-//           blocks, each an FMA chain from +0, added in order):
-//           q4a_rows_chain, a thread per (row, token),
-//           where K and g are multiples of 32, else q4a_gemm_rows.
+//           blocks, each an FMA chain from +0, added in order), on the f32
+//           matrix cores (mm_f32.hip).
 // Both bit-exact to the oracle.
 //
 // M == 1 layout of the work: the groups of a row are independent until the
@@ -140,110 +139,6 @@ __global__ __launch_bounds__(QT) void q4a_gemv_kernel(const uint8_t* __restrict_
     for (int r = threadIdx.x; r < nr; r += QT) out[r0 + r] = lds_seq_sum(cg + r * ngp, ng, 0.0f);
 }
 
-// M > 1: one thread per output column j and up to MT token rows.
-template <int MT>
-__global__ __launch_bounds__(QT) void q4a_gemm_rows(const uint8_t* __restrict__ packed, size_t pitch,
-                                                    const uint32_t* __restrict__ sm, int N, int K, int g,
-                                                    const float* __restrict__ a, int M, float* __restrict__ out) {
-    const int j = blockIdx.x * QT + threadIdx.x;
-    const int m0 = blockIdx.y * MT;
-    if (j >= N) return;
-    const int ng = (K + g - 1) / g;
-    const uint8_t* prow = packed + (size_t)j * pitch;
-    const uint32_t* srow = sm + (size_t)j * ng;
-    float acc[MT], tot[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) tot[m] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += MM_KC) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = 0.0f;
-        for (int kk = k0; kk < min(K, k0 + MM_KC); ++kk) {
-            const uint8_t byte = prow[kk >> 1];
-            const uint32_t s = srow[kk / g];
-            const float w = h2f((uint16_t)(s & 0xffffu)) * (float)((kk & 1) ? (byte >> 4) : (byte & 15)) +
-                            h2f((uint16_t)(s >> 16));
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                if (m0 + m < M) acc[m] = __builtin_fmaf(a[(size_t)(m0 + m) * K + kk], w, acc[m]);
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m) tot[m] = tot[m] + acc[m];
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-        if (m0 + m < M) out[(size_t)(m0 + m) * N + j] = tot[m];
-}
-
-// M > 1 with K % 32 == 0, g % 32 == 0 and 16-byte aligned activation rows:
-// one thread per (column j, token row blockIdx.y), the packed row read 16
-// bytes (32 nibbles) and the token's 32 activations (uniform across the
-// workgroup) at a time, one chunk ahead of the chain.  The order per output
-// is q4a_gemm_rows' (a.dot's blocks over kk, w = scale * q + min), bit for
-// bit.
-__global__ __launch_bounds__(QT) void q4a_rows_chain(const uint8_t* __restrict__ packed, size_t pitch,
-                                                     const uint32_t* __restrict__ sm, int N, int K, int g,
-                                                     const float* __restrict__ a, float* __restrict__ out) {
-    const int j = blockIdx.x * QT + threadIdx.x, m = blockIdx.y;
-    const int jj = min(j, N - 1);  // clamped: the loads stay unconditional, the store is guarded
-    const int nc = K / 32, ng = K / g;
-    const uint4* prow = reinterpret_cast<const uint4*>(packed + (size_t)jj * pitch);
-    const uint32_t* srow = sm + (size_t)jj * ng;
-    const float4* arow = reinterpret_cast<const float4*>(a + (size_t)m * K);
-    struct Chunk {
-        uint4 w;
-        uint32_t s;
-        float4 av[8];
-    };
-    auto ld = [&](Chunk& c, int i) {
-        c.w = prow[i];
-        c.s = srow[(32 * i) / g];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) c.av[u] = arow[8 * i + u];
-    };
-    float acc = 0.0f;
-    auto chain = [&](const Chunk& c) {
-        const uint32_t ws[4] = {c.w.x, c.w.y, c.w.z, c.w.w};
-        const float sc = h2f((uint16_t)(c.s & 0xffffu)), mn = h2f((uint16_t)(c.s >> 16));
-#pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4) {
-            const float x[8] = {c.av[2 * c4].x, c.av[2 * c4].y, c.av[2 * c4].z, c.av[2 * c4].w,
-                                c.av[2 * c4 + 1].x, c.av[2 * c4 + 1].y, c.av[2 * c4 + 1].z, c.av[2 * c4 + 1].w};
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                acc = __builtin_fmaf(x[q], sc * (float)((ws[c4] >> (4 * q)) & 15u) + mn, acc);
-        }
-    };
-    // a.dot's blocks: MM_KC / 32 chunks (an even count) each, folded in
-    // where a block starts (an even chunk)
-    static_assert(MM_KC % 64 == 0, "blocks start on even chunks");
-    float tot = 0.0f;
-    auto fold = [&](int i) {
-        if (i > 0 && i % (MM_KC / 32) == 0) {
-            tot = tot + acc;
-            acc = 0.0f;
-        }
-    };
-    Chunk c0, c1;
-    ld(c0, 0);
-    ld(c1, min(1, nc - 1));
-    __builtin_amdgcn_sched_barrier(0);
-    int i = 0;
-    for (; i + 2 <= nc; i += 2) {
-        fold(i);
-        chain(c0);
-        ld(c0, min(i + 2, nc - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        chain(c1);
-        ld(c1, min(i + 3, nc - 1));
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (i < nc) {
-        fold(i);
-        chain(c0);
-    }
-    if (j < N) out[(size_t)m * N + j] = tot + acc;
-}
-
 }  // namespace
 
 size_t q4a_pitch(size_t k) { return round_up((k + 1) / 2, 16); }
@@ -273,15 +168,17 @@ hipError_t launch_q4a(const Weight& w, size_t m, const float* a, float* out, hip
                                                                 (int)w.g, rb, a, out);
         return hipGetLastError();
     }
-    if (w.k % 32 == 0 && w.g % 32 == 0 && ((uintptr_t)a & 15) == 0 && m <= 65535) {
-        q4a_rows_chain<<<dim3((unsigned)((w.n + QT - 1) / QT), (unsigned)m), dim3(QT), 0, s>>>(
-            w.q4raw, w.rpitch, w.q4a_sm, (int)w.n, (int)w.k, (int)w.g, a, out);
-        return hipGetLastError();
-    }
-    dim3 grid((unsigned)((w.n + QT - 1) / QT), (unsigned)((m + 15) / 16));
-    q4a_gemm_rows<16><<<grid, dim3(QT), 0, s>>>(w.q4raw, w.rpitch, w.q4a_sm, (int)w.n, (int)w.k, (int)w.g, a, (int)m,
-                                                 out);
-    return hipGetLastError();
+    MmWeight v{};
+    v.w = w.q4raw;
+    v.sc = reinterpret_cast<const uint16_t*>(w.q4a_sm);
+    v.mn = v.sc + 1;
+    v.ss = 2;
+    v.n = (int)w.n;
+    v.k = (int)w.k;
+    v.g = (int)std::min(w.g, std::max<size_t>(w.k, 1));  // a longer group is one group
+    v.ng = ng;
+    v.pitch = w.rpitch;
+    return launch_mm_f32(FRQ_DT_Q4A, v, a, m, out, device_cus(w.device), s);
 }
 
 }  // namespace frq
