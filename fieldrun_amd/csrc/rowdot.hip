@@ -43,6 +43,16 @@ __device__ __forceinline__ unsigned long long argmax_key(float v, int row) {
     return ((unsigned long long)u << 32) | (uint32_t)row;
 }
 
+// f(0), ..., f(N - 1) with constant arguments (register arrays indexed by
+// them stay in registers whatever f's size).
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void unrolled(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unrolled<N, I + 1>(f);
+    }
+}
+
 // NX x vectors at once (outputs out + v os, argmax best[v], v < nv): each
 // lane runs NX chains of its row, one per vector, so the table streams once
 // for all of them; every chain is the one-vector order.  For NX > 1, x is
@@ -186,29 +196,15 @@ __global__ __launch_bounds__(64 * WPB) void rowdot_kernel(
     // is issued unconditionally (the index clamped to the last chunk, whose
     // re-reads hit L2), so the waits before a buffer's use count exactly
     // the loads issued after it.
-    uint4 b0[8], b1[8], b2[8];
+    uint4 b[DEPTH][8];
     if (nch > 0) {
         const int last = nch - 1;
-        load(b0, 0);
-        load(b1, min(1, last));
-        if constexpr (DEPTH == 2) {
-            for (int c = 0; c < nch; c += 2) {
-                consume(b0, c);
-                load(b0, min(c + 2, last));
-                if (c + 1 < nch) consume(b1, c + 1);
-                load(b1, min(c + 3, last));
-            }
-        } else {
-            load(b2, min(2, last));
-            for (int c = 0; c < nch; c += 3) {
-                consume(b0, c);
-                load(b0, min(c + 3, last));
-                if (c + 1 < nch) consume(b1, c + 1);
-                load(b1, min(c + 4, last));
-                if (c + 2 < nch) consume(b2, c + 2);
-                load(b2, min(c + 5, last));
-            }
-        }
+        unrolled<DEPTH>([&](auto j) { load(b[j], min((int)j, last)); });
+        for (int c = 0; c < nch; c += DEPTH)
+            unrolled<DEPTH>([&](auto j) __attribute__((always_inline)) {
+                if (j == 0 || c + j < nch) consume(b[j], c + j);
+                load(b[j], min(c + j + DEPTH, last));
+            });
     }
     const int o = o0 + lane;
 #pragma unroll
@@ -237,69 +233,67 @@ __global__ __launch_bounds__(64 * WPB) void rowdot_kernel(
 template <int DT, bool ARG>
 hipError_t launch_dt(const Weight& w, const float* x, const int64_t* cand, size_t nout, float* out,
                      unsigned long long* best, int* err, hipStream_t s) {
-    // fewer waves than about four per SIMD: keep three chunks in flight per
-    // wave (latency-bound), else two (the occupancy carries the load)
-    const bool deep = nout < 4 * 1024 * 64;
-    const unsigned g4 = (unsigned)((nout + 255) / 256);
+    // At most one wave a SIMD: workgroups of one wave, over all the CUs, and
+    // six chunks in flight (16384 x 3584 f16: 64 -> 48 us; four-wave
+    // workgroups leave three CUs in four idle there).  Up to about four waves
+    // per SIMD: three chunks (latency-bound), else two (the occupancy carries
+    // the load).
+    const bool few = nout <= 1024 * 64, deep = nout < 4 * 1024 * 64;
 #define FRQ_ROWDOT(SUBV, DEPTHV, WPBV)                                                                   \
-    rowdot_kernel<DT, SUBV, DEPTHV, WPBV, ARG><<<dim3(g4), dim3(64 * WPBV), 0, s>>>(                   \
-        w.rowp, w.scale, (int)w.n, (int)w.k, w.rpitch, x, cand, (int)nout, out, best, err)
+    rowdot_kernel<DT, SUBV, DEPTHV, WPBV, ARG>                                                           \
+        <<<dim3((unsigned)((nout + 64 * WPBV - 1) / (64 * WPBV))), dim3(64 * WPBV), 0, s>>>(             \
+            w.rowp, w.scale, (int)w.n, (int)w.k, w.rpitch, x, cand, (int)nout, out, best, err)
     if (cand) {
-        if (deep) FRQ_ROWDOT(true, 3, 4);
+        if (few) FRQ_ROWDOT(true, 6, 1);
+        else if (deep) FRQ_ROWDOT(true, 3, 4);
         else FRQ_ROWDOT(true, 2, 4);
     } else {
-        if (deep) FRQ_ROWDOT(false, 3, 4);
+        if (few) FRQ_ROWDOT(false, 6, 1);
+        else if (deep) FRQ_ROWDOT(false, 3, 4);
         else FRQ_ROWDOT(false, 2, 4);
     }
 #undef FRQ_ROWDOT
     return hipGetLastError();
 }
 
-// Products w * x[u] for vectors u = U, U + 1 of one element: x (a VGPR)
-// holds vector u's value in lane u of each 16-lane DPP row, and
-// v_mul_f32_dpp row_newbcast:u hands every lane that value times its own w.
-// NOP: the two wait states a DPP read needs after a VALU write of x (the
-// compiler does not see into the asm).
-#define FRQ_DPPM(dst, n) "v_mul_f32_dpp %" #dst ", %2, %3 row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
-template <int U, bool NOP>
-__device__ __forceinline__ void dpp_mul2(float& p0, float& p1, float x, float w) {
-    static_assert(U >= 0 && U <= 14 && U % 2 == 0, "lane pair");
-#define FRQ_DPPM_CASE(u0, u1)                                                                        \
-    if constexpr (U == u0) {                                                                         \
-        if constexpr (NOP) asm("s_nop 1\n\t" FRQ_DPPM(0, u0) FRQ_DPPM(1, u1) : "=&v"(p0), "=&v"(p1) : "v"(x), "v"(w)); \
-        else asm(FRQ_DPPM(0, u0) FRQ_DPPM(1, u1) : "=&v"(p0), "=&v"(p1) : "v"(x), "v"(w));              \
-    }
-    FRQ_DPPM_CASE(0, 1) FRQ_DPPM_CASE(2, 3) FRQ_DPPM_CASE(4, 5) FRQ_DPPM_CASE(6, 7)
-    FRQ_DPPM_CASE(8, 9) FRQ_DPPM_CASE(10, 11) FRQ_DPPM_CASE(12, 13) FRQ_DPPM_CASE(14, 15)
-#undef FRQ_DPPM_CASE
-}
-#undef FRQ_DPPM
+typedef float f4v __attribute__((ext_vector_type(4)));
 
 // The f32 / f16 fold for 2 <= NX <= 16 vectors with the argmax (the
 // batched head): each output is rowdot_kernel's fold (acc = acc + w * x
 // from -0.0, k ascending).  A lane owns a row (read from the LDS tile 16
-// bytes at a time); an element's NX products come from dpp_mul2 (x
-// broadcast from a register, no scalar loads: their latency, not the
-// arithmetic, bounded the scalar-x form), then its NX adds.  x is in the
-// k-quad interleaved layout xq[64 (k / 4) + 4 v + k % 4] (16 vector slots,
-// k < d + 4; lane l loads the quad of vector l % 16), one quad ahead.  The
-// next chunk's row tile loads into the registers the current one was
-// staged from.
-template <int DT, int NX>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rowdot_nx_kernel(const uint8_t* __restrict__ W, int rows, int d, size_t pitch,
+// bytes at a time); an element's products with four vectors are one
+// v_mfma_f32_4x4x1_16b on -0 (fma(w, x, -0) is w * x in one rounding, its
+// sign with it): block b's columns are the rows of lanes 4 b .. 4 b + 3, its
+// rows the four vectors, so lane l holds its row's product with vector v in
+// element v, 8 clocks against 32 for four DPP-broadcast multiplies; then the
+// adds.  x is in the k-quad interleaved layout xq[64 (k / 4) + 4 v + k % 4]
+// (16 vector slots, k < d + 4), a chunk's quads staged in LDS with its row
+// tile (loaded quad by quad they waited for the table's loads issued before
+// them: 124 against 86 us, 16 vectors x 16384 x 2304 f16).
+// VS waves of a workgroup take the same 64 rows and four vectors each (a
+// table of few rows fills the SIMDs so; eight vectors a wave were slower at
+// every size).  Bound by the adds, the products and the LDS reads.  Against
+// DPP-broadcast products and all vectors in one wave, 16 vectors: 16384 x
+// 2304 f16 287 -> 86 us, 256000 x 2304 770 -> 659; 4 vectors 397 -> 320.
+template <int DT, int VS>
+__global__ __launch_bounds__(256, 4) void rowdot_nx_kernel(const uint8_t* __restrict__ W, int rows, int d, size_t pitch,
                                                         const float* __restrict__ xq, float* __restrict__ out,
                                                         unsigned long long* __restrict__ best, int* __restrict__ err,
                                                         size_t os, int nv) {
     static_assert(DT == 0 || DT == 1, "the fold arms");
-    static_assert(NX >= 2 && NX <= 16 && NX % 2 == 0, "vector pairs");
+    constexpr int NX = 4;  // vectors a wave: one MFMA's
+    static_assert(VS == 1 || VS == 2 || VS == 4, "waves of a workgroup on the same rows");
     constexpr int ES = DT == 0 ? 4 : 2;  // bytes per element
     constexpr int EQ = 16 / ES;          // elements per 16-byte piece
     __shared__ __attribute__((aligned(16))) uint8_t tile[4][64 * TP];
+    __shared__ f4v xs[4][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int o0 = ((int)blockIdx.x * 4 + wave) * 64;
-    if (o0 >= rows) return;  // wave-uniform; no block-wide barrier below
+    const int o0 = ((int)blockIdx.x * (4 / VS) + wave / VS) * 64;
+    const int v0 = NX * (wave % VS);  // this wave's first vector
+    if (o0 >= rows || v0 >= nv) return;  // wave-uniform; no block-wide barrier below
     uint8_t* tw = tile[wave];
+    f4v* xw = xs[wave];  // a chunk's x: quad, vector
     // load instruction i of a chunk: row o0 + 8 i + lane / 8 (the last row
     // past the end), bytes 16 (lane % 8); 32-bit offsets from the wave's
     // first row (64 rows of one table)
@@ -309,69 +303,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
     for (int i = 0; i < 8; ++i)
         lo[i] = (uint32_t)min(8 * i + (lane >> 3), rows - 1 - o0) * (uint32_t)pitch + (lane & 7) * 16;
     const int nch = (int)(pitch / 128);
-    const float* xl = xq + 4 * (lane & 15);
+    const float* xl = xq + 4 * (v0 + (lane & 3));  // a chunk's x: lane 4 q + v loads quad q of vector v
     const int nq = (d + 3) / 4;  // quads of x
-    float acc[NX];
-#pragma unroll
-    for (int u = 0; u < NX; ++u) acc[u] = -0.0f;
+    f4v acc = {-0.0f, -0.0f, -0.0f, -0.0f};
     // element e of piece q (a uint4 of the lane's row) as f32
     auto elem = [&](const uint4& q, int e) __attribute__((always_inline)) -> float {
         const uint32_t wd = e / (4 / ES) == 0 ? q.x : e / (4 / ES) == 1 ? q.y : e / (4 / ES) == 2 ? q.z : q.w;
         if constexpr (DT == 0) return __builtin_bit_cast(float, wd);
         else return h2f((uint16_t)(wd >> (16 * (e & 1))));
     };
-    // one element: w times its x (component i of the quad xv); ADD: k < d
-    auto fold = [&](float w, const float4& xv, int i, bool add) __attribute__((always_inline)) {
-        const float xi = i == 0 ? xv.x : i == 1 ? xv.y : i == 2 ? xv.z : xv.w;
-        float pr[NX];
-        dpp_mul2<0, true>(pr[0], pr[1], xi, w);
-        if constexpr (NX > 2) dpp_mul2<2, false>(pr[2], pr[3], xi, w);
-        if constexpr (NX > 4) {
-            dpp_mul2<4, false>(pr[4], pr[5], xi, w);
-            dpp_mul2<6, false>(pr[6], pr[7], xi, w);
-        }
-        if constexpr (NX > 8) {
-            dpp_mul2<8, false>(pr[8], pr[9], xi, w);
-            dpp_mul2<10, false>(pr[10], pr[11], xi, w);
-            dpp_mul2<12, false>(pr[12], pr[13], xi, w);
-            dpp_mul2<14, false>(pr[14], pr[15], xi, w);
-        }
+    // one element: w times its x (component i of the quad xv); add: k < d
+    const f4v nz = {-0.0f, -0.0f, -0.0f, -0.0f};
+    auto fold = [&](float w, const f4v& xv, int i, bool add) __attribute__((always_inline)) {
+        const f4v pr = __builtin_amdgcn_mfma_f32_4x4x1f32(xv[i], w, nz, 0, 0, 0);
         if (add) {
 #pragma unroll
-            for (int u = 0; u < NX; ++u) acc[u] = acc[u] + pr[u];
+            for (int v = 0; v < 4; ++v) acc[v] = acc[v] + pr[v];
         }
     };
-    auto xload = [&](int kq) __attribute__((always_inline)) {
-        return *reinterpret_cast<const float4*>(xl + (size_t)min(kq, nq - 1) * 64);
-    };
-    // a chunk's elements k0 .. k0 + 128 / ES; CHECK: only k < d.  The quads
-    // alternate two register sets (an even count a chunk).
-    float4 xa = xload(0), xb;
+    // a chunk's elements k0 .. k0 + 128 / ES; CHECK: only k < d
     auto run = [&](auto check, int k0) __attribute__((always_inline)) {
         constexpr bool CHECK = decltype(check)::value;
-        const int kq0 = k0 / 4;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        unrolled<8>([&](auto j) __attribute__((always_inline)) {
             const uint4 q = *reinterpret_cast<const uint4*>(tw + lane * TP + 16 * j);
-#pragma unroll
-            for (int h = 0; h < EQ / 4; ++h) {
-                const int qi = j * (EQ / 4) + h;  // quad of the chunk
-                if (qi % 2 == 0) {
-                    xb = xload(kq0 + qi + 1);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) fold(elem(q, 4 * h + i), xa, i, !CHECK || k0 + 4 * qi + i < d);
-                } else {
-                    xa = xload(kq0 + qi + 1);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) fold(elem(q, 4 * h + i), xb, i, !CHECK || k0 + 4 * qi + i < d);
-                }
-            }
-        }
+            unrolled<EQ / 4>([&](auto h) __attribute__((always_inline)) {
+                constexpr int qi = j * (EQ / 4) + h;  // quad of the chunk
+                const f4v xv = xw[qi * 4 + (lane & 3)];
+                unrolled<4>([&](auto i) __attribute__((always_inline)) {
+                    fold(elem(q, 4 * h + i), xv, i, !CHECK || k0 + 4 * qi + i < d);
+                });
+            });
+        });
     };
     uint4 b[8];
+    f4v bx;
     auto load = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) b[i] = ntload16u(wb + (size_t)c * 128 + lo[i]);
+        bx = *reinterpret_cast<const f4v*>(xl + 64 * (size_t)min(c * (32 / ES) + (lane >> 2), nq - 1));
     };
     if (nch > 0) {
         load(0);
@@ -379,6 +348,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 *reinterpret_cast<uint4*>(tw + (8 * i + (lane >> 3)) * TP + (lane & 7) * 16) = b[i];
+            xw[lane] = bx;
             load(min(c + 1, nch - 1));  // the next chunk, under this one's arithmetic
             wave_sync();
             const int k0 = c * (128 / ES);
@@ -390,9 +360,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
     const int o = o0 + lane;
 #pragma unroll
     for (int u = 0; u < NX; ++u) {
-        if (u >= nv) break;  // the zero padding of the transposed x
+        if (v0 + u >= nv) break;  // the zero padding of the transposed x
         const float a = acc[u];
-        if (o < rows) out[u * os + o] = a;
+        if (o < rows) out[(size_t)(v0 + u) * os + o] = a;
         unsigned long long key = o < rows ? argmax_key(a, o) : 0ull;
         const bool nan = o < rows && a != a;
 #pragma unroll
@@ -401,7 +371,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
             key = ok > key ? ok : key;
         }
         if (__builtin_amdgcn_ballot_w64(nan) && lane == 0) atomicOr(err, 1);
-        if (lane == 0) atomicMax(best + u, key);
+        if (lane == 0) atomicMax(best + v0 + u, key);
     }
 }
 
@@ -433,8 +403,9 @@ hipError_t launch_argmax_nx(const Weight& w, size_t nv, const float* x, size_t x
     if constexpr (NX > 1 && DT != 2) {
         const size_t nq = (w.k + 3) / 4;
         quad_x_kernel<<<dim3((unsigned)((nq * 64 + 255) / 256)), dim3(256), 0, s>>>(x, xs, (int)nv, (int)w.k, xt);
-        rowdot_nx_kernel<DT, NX><<<dim3(g4), dim3(256), 0, s>>>(w.rowp, (int)w.n, (int)w.k, w.rpitch, xt, out, best,
-                                                                 err, os, (int)nv);
+        constexpr int VS = NX <= 4 ? 1 : NX / 4, RW = 64 * (4 / VS);  // RW: rows a workgroup
+        rowdot_nx_kernel<DT, VS><<<dim3((unsigned)((w.n + RW - 1) / RW)), dim3(256), 0, s>>>(
+            w.rowp, (int)w.n, (int)w.k, w.rpitch, xt, out, best, err, os, (int)nv);
     } else {
         const float* xv = x;
         if constexpr (NX > 1) {
