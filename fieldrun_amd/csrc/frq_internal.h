@@ -538,6 +538,10 @@ size_t i4_ws_floats(const Weight& w, size_t m);
 // int4 at M == 1 in i4_dot_avx2's order (bit-exact) with coalesced loads, for
 // K % 32 == 0 and g in {32, 64}; hipErrorNotSupported for other shapes.
 hipError_t launch_i4_terms(const Weight& w, const float* a, float* out, hipStream_t s);
+// One row through packed int4 (q4a: affine, with mins) rows of any K and
+// group, in the AVX2 order; sc / mn ss apart.
+hipError_t launch_pack_m1_any(bool q4a, const uint8_t* packed, size_t pitch, const uint16_t* sc, const uint16_t* mn,
+                              int ss, size_t n, size_t k, size_t g, const float* a, float* out, hipStream_t s);
 // int4 in the reference's orders for any m (M == 1 i4_dot_avx2, M > 1 the
 // dequantise + sequential-k GEMM): the paths decode engines use.
 hipError_t launch_i4_exact(const Weight& w, size_t m, const float* a, float* out, hipStream_t s);

@@ -92,6 +92,60 @@ __global__ void i4_gemv_generic(const uint8_t* __restrict__ packed,
     out[j] = sum;
 }
 
+// M == 1 for any K and g (int4 in i4_dot_avx2's order, Q: q4a in
+// q4a_dot_avx2's): a thread a (row, group), adjacent threads adjacent groups,
+// the packed words read eight nibbles at a time at whatever byte they start,
+// the activation row in LDS (36 floats a 32, so lanes a group apart meet
+// other banks), and a lane a row adding its group terms in order.  Bound by
+// the VALU at wide outputs and by the latency of a group's chain at narrow
+// ones; a thread a row instead (i4_gemv_generic, kept where LDS does not hold
+// the row and its terms) walks all of K alone: 184 x 6346 334 -> 8 us.
+__device__ __forceinline__ int any_pad(int k) { return k + (k >> 5) * 4; }
+
+template <bool Q>
+__global__ __launch_bounds__(256) void pack_gemv_any(const uint8_t* __restrict__ packed, size_t pitch,
+                                                     const uint16_t* __restrict__ sc, const uint16_t* __restrict__ mn,
+                                                     int ss, int N, int K, int g, int rb,
+                                                     const float* __restrict__ a, float* __restrict__ out) {
+    typedef uint32_t word_u __attribute__((aligned(1)));
+    extern __shared__ float4 any_lds[];
+    float* as = reinterpret_cast<float*>(any_lds);
+    const int ng = (K + g - 1) / g, ngp = (ng + 3) & ~3;
+    float* cg = as + (any_pad(K) + 7) / 4 * 4;
+    const int r0 = blockIdx.x * rb, nr = min(rb, N - r0), items = nr * ng;
+    for (int i = threadIdx.x; i < K; i += 256) as[any_pad(i)] = a[i];
+    __syncthreads();
+    for (int p = threadIdx.x; p < items; p += 256) {
+        const int r = p / ng, gi = p - r * ng;
+        const uint8_t* prow = packed + (size_t)(r0 + r) * pitch;
+        int kk = gi * g;
+        const int hi = min(kk + g, K);
+        float l[8] = {0, 0, 0, 0, 0, 0, 0, 0}, m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (; kk + 8 <= hi; kk += 8) {
+            const uint32_t w = *reinterpret_cast<const word_u*>(prow + (kk >> 1));  // from an even index on
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const float av = as[any_pad(kk + q)];
+                const float wv = Q ? (float)((w >> (4 * q)) & 15u) : s4f(w, q);
+                l[q] = __builtin_fmaf(wv, av, l[q]);
+                if (Q) m[q] = m[q] + av;
+            }
+        }
+        float qs = ((l[0] + l[4]) + (l[2] + l[6])) + ((l[1] + l[5]) + (l[3] + l[7]));
+        float ms = ((m[0] + m[4]) + (m[2] + m[6])) + ((m[1] + m[5]) + (m[3] + m[7]));
+        for (; kk < hi; ++kk) {
+            const int v = (kk & 1) ? prow[kk >> 1] >> 4 : prow[kk >> 1] & 15;
+            const float av = as[any_pad(kk)];
+            qs = qs + av * (float)(Q ? v : (v ^ 8) - 8);
+            if (Q) ms = ms + av;
+        }
+        const size_t at = ((size_t)(r0 + r) * ng + gi) * ss;
+        cg[r * ngp + gi] = Q ? h2f(sc[at]) * qs + h2f(mn[at]) * ms : h2f(sc[at]) * qs;
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < nr; r += 256) out[r0 + r] = lds_seq_sum(cg + r * ngp, ng, 0.0f);
+}
+
 // M == 1 in i4_dot_avx2's order, fast: a group's term scale * gsum is
 // independent of the others until the in-order sum, so a thread takes one
 // (row, group) at a time (adjacent threads adjacent groups: the G4 16-byte
@@ -1155,7 +1209,39 @@ hipError_t launch_i4_m1_rows(const Weight& w, size_t m, const float* a, float* o
     return hipSuccess;
 }
 
+// Any K and g at M == 1; hipErrorNotSupported where a row's activations and
+// terms exceed 64 KB of LDS.  Rows a workgroup: as many as fit beside the
+// activations, fewer while the grid is short and a row still fills half the
+// threads.
+hipError_t launch_pack_m1_any(bool q4a, const uint8_t* packed, size_t pitch, const uint16_t* sc, const uint16_t* mn,
+                              int ss, size_t n, size_t k, size_t g, const float* a, float* out, hipStream_t s) {
+    if (k == 0 || g == 0 || n > (size_t)INT32_MAX || k > 16384) return hipErrorNotSupported;
+    const size_t gg = std::min(g, k), ng = (k + gg - 1) / gg, row = ((ng + 3) & ~(size_t)3) * 4;
+    const size_t act = ((k + k / 32 * 4) / 4 + 4) * 16;
+    if (act + row > 64 * 1024) return hipErrorNotSupported;
+    size_t rb = std::min<size_t>(64, (64 * 1024 - act) / row);
+    while (rb > 1 && (n + rb - 1) / rb < 512 && rb * ng > 256) rb = (rb + 1) / 2;
+    const unsigned grid = (unsigned)((n + rb - 1) / rb);
+    const size_t lds = act + rb * row;
+    if (q4a)
+        pack_gemv_any<true><<<dim3(grid), dim3(256), lds, s>>>(packed, pitch, sc, mn, ss, (int)n, (int)k, (int)gg,
+                                                               (int)rb, a, out);
+    else
+        pack_gemv_any<false><<<dim3(grid), dim3(256), lds, s>>>(packed, pitch, sc, mn, ss, (int)n, (int)k, (int)gg,
+                                                                (int)rb, a, out);
+    return hipGetLastError();
+}
+
 namespace {
+hipError_t i4_m1_any(const Weight& w, const float* a, float* out, hipStream_t s) {
+    const hipError_t e = launch_pack_m1_any(false, w.q4raw, (w.k + 1) / 2, w.s4raw, nullptr, 1, w.n, w.k, w.g, a,
+                                            out, s);
+    if (e != hipErrorNotSupported) return e;
+    i4_gemv_generic<<<dim3((unsigned)((w.n + 255) / 256)), dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k,
+                                                                             (int)w.g, a, out);
+    return hipGetLastError();
+}
+
 // M > 1: the dequantised weights on the f32 matrix cores, in a.dot's order.
 hipError_t mm_dequant(const Weight& w, size_t m, const float* a, float* out, hipStream_t s) {
     if (w.n > (size_t)INT32_MAX || w.k > (size_t)INT32_MAX) return hipErrorInvalidValue;
@@ -1177,9 +1263,7 @@ hipError_t launch_i4_exact(const Weight& w, size_t m, const float* a, float* out
     if (m == 1) {
         const hipError_t e = launch_i4_terms(w, a, out, s);
         if (e != hipErrorNotSupported) return e;
-        i4_gemv_generic<<<dim3((unsigned)((w.n + 255) / 256)), dim3(256), 0, s>>>(
-            w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, out);
-        return hipGetLastError();
+        return i4_m1_any(w, a, out, s);
     }
     return mm_dequant(w, m, a, out, s);
 }
@@ -1208,11 +1292,7 @@ hipError_t launch_i4(const Weight& w, size_t m, const float* a, float* out,
             default: return launch_mfma<4>(w, m, a, adig, sog, out, s);
         }
     }
-    if (m == 1) {
-        i4_gemv_generic<<<dim3((unsigned)((w.n + 255) / 256)), dim3(256), 0, s>>>(
-            w.q4raw, w.s4raw, (int)w.n, (int)w.k, (int)w.g, a, out);
-        return hipGetLastError();
-    }
+    if (m == 1) return i4_m1_any(w, a, out, s);
     return mm_dequant(w, m, a, out, s);
 }
 

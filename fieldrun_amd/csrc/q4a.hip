@@ -163,9 +163,13 @@ hipError_t launch_q4a(const Weight& w, size_t m, const float* a, float* out, hip
         else if (vec)
             q4a_gemv_kernel<2><<<dim3(grid), dim3(QT), cgb + asb, s>>>(w.q4raw, w.rpitch, w.q4a_sm, (int)w.n,
                                                                       (int)w.k, (int)w.g, rb, a, out);
-        else
+        else {
+            const uint16_t* sc = reinterpret_cast<const uint16_t*>(w.q4a_sm);
+            const hipError_t e = launch_pack_m1_any(true, w.q4raw, w.rpitch, sc, sc + 1, 2, w.n, w.k, w.g, a, out, s);
+            if (e != hipErrorNotSupported) return e;
             q4a_gemv_kernel<0><<<dim3(grid), dim3(QT), cgb, s>>>(w.q4raw, w.rpitch, w.q4a_sm, (int)w.n, (int)w.k,
                                                                 (int)w.g, rb, a, out);
+        }
         return hipGetLastError();
     }
     MmWeight v{};

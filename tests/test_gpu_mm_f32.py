@@ -82,3 +82,18 @@ def test_expert_banks_in_a_dot_order(ctx, dtype, T, topk, d, mi):
     lg = rng.standard_normal((T, E)).astype(np.float32)
     per_row = np.stack([bank.forward(x[t:t + 1], lg[t:t + 1], topk)[0] for t in range(T)])
     same(bank.forward(x, lg, topk), per_row)  # tiles of 4 and of 32 rows, one expert's rows alone or together
+
+
+@pytest.mark.parametrize("g", [32, 64, 13, 1, 4000])
+@pytest.mark.parametrize("k,n", [(1, 3), (31, 5), (33, 300), (255, 64), (790, 1), (1001, 700), (6346, 184), (2304, 129),
+                                 (16383, 17), (16400, 9)])
+def test_one_row_of_any_width_and_group(ctx, k, n, g):
+    """M == 1 where the aligned kernels do not apply: the AVX2 orders, groups
+    that start inside a byte, rows too long for LDS."""
+    rng = np.random.default_rng(k + n + g)
+    a = rng.standard_normal((1, k), dtype=np.float32)
+    q, s, mn = packed_weight(rng, n, k, g)
+    same(ctx.upload_i4(q, s, k, g).mm_exact(a), oracle.mm_i4(a, q, s.astype(np.float32), k, g))
+    if (k + g - 1) // g <= 8192:  # q4a: one row's group terms must fit in LDS
+        same(ctx.upload_q4a(q, s, mn, k, g).mm(a),
+             oracle.mm_q4a(a, q, s.astype(np.float32), mn.astype(np.float32), k, g))
