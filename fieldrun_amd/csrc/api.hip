@@ -6,6 +6,8 @@
 //   int8, M == 1           -> fused quant + GEMV (one launch)
 //   int8, 2 <= M <= 16     -> quant kernel + skinny MFMA kernel (weights
 //                             streamed once; bit-exact epilogue)
+//   int8, M > 16, small    -> quant kernel + mid kernel (a wave a 16-row tile;
+//                             bit-exact epilogue)
 //   int8, M >  16          -> quant kernel (blocked a8) + int8 MFMA GEMM
 //   int4                   -> blocked W4A32 GEMV (M == 1) / batched kernel
 // Every failure becomes an int status plus frq_last_error(); nothing throws.
@@ -119,11 +121,17 @@ struct Carve {
     }
 };
 
-// Decode batches (m <= 16) take the row-major a8 and the HBM-bound kernels;
-// larger m the blocked a8 and the MFMA GEMM.
-bool use_gemv(const Weight& w, size_t m) {
-    (void)w;
-    return m <= 16;
+// Decode batches (m <= 16) and the middling batches of mid_i8_ok take the
+// row-major a8 and the kernels that form their outputs in one pass; larger m
+// the blocked a8 and the MFMA GEMM.
+bool use_gemv(const Weight& w, size_t m) { return m <= 16 || mid_i8_ok(w, m); }
+
+// The int8 dot and epilogue on a row-major a8 (use_gemv).
+hipError_t launch_rows_i8(const Weight& w, size_t m, const int8_t* a8, const float* sa, const uint32_t* oi,
+                          const float* ov, float* out, int32_t* acc, hipStream_t s) {
+    if (m == 1) return launch_gemv_i8(w, m, a8, sa, oi, ov, out, acc, s);
+    if (m <= 16) return launch_skinny_i8(w, m, a8, sa, oi, ov, out, acc, s);
+    return launch_mid_i8(w, m, a8, sa, oi, ov, out, acc, s);
 }
 
 // Bytes of per-call scratch for an int8 linear of m rows (a second, row-major
@@ -162,10 +170,7 @@ int run_i8(frq_ctx* c, const Weight& w, const float* d_a, size_t m, float* d_out
                "launch linear_m1");
     } else if (!gemm) {
         HIPCHK(launch_quant(d_a, m, w.k, w.kp, a8, sa, oi, ov, c->err, c->stream), "launch quant");
-        if (m == 1)
-            HIPCHK(launch_gemv_i8(w, m, a8, sa, oi, ov, d_out, d_acc, c->stream), "launch gemv_i8");
-        else
-            HIPCHK(launch_skinny_i8(w, m, a8, sa, oi, ov, d_out, d_acc, c->stream), "launch skinny_i8");
+        HIPCHK(launch_rows_i8(w, m, a8, sa, oi, ov, d_out, d_acc, c->stream), "launch rows_i8");
     } else {
         HIPCHK(launch_quant(d_a, m, w.k, w.kp, a8, sa, oi, ov, c->err, c->stream, mp), "launch quant");
         HIPCHK(launch_gemm_i8(w, m, a8, sa, oi, ov, d_out, d_acc, gws, c->stream), "launch gemm_i8");
@@ -177,8 +182,7 @@ int run_i8(frq_ctx* c, const Weight& w, const float* d_a, size_t m, float* d_out
 
 bool rows_exact_ok(const frq_w* wh, size_t m) {
     const Weight& w = wh->w;
-    return w.dtype == FRQ_DT_I8 && m > 16 && m <= 65535 && w.k > 0 && w.wblk && w.wkn && w.kp <= 20480 &&
-           !use_gemv(w, m);
+    return w.dtype == FRQ_DT_I8 && m > 16 && m <= 65535 && w.k > 0 && w.wblk && w.wkn && w.kp <= 20480;
 }
 
 int rows_exact(frq_ctx* c, const frq_w* wh, const float* d_a, size_t m, float* d_out) {
@@ -193,6 +197,11 @@ int rows_exact(frq_ctx* c, const frq_w* wh, const float* d_a, size_t m, float* d
     float* sa = cv.take<float>(mp);
     uint32_t* oi = cv.take<uint32_t>(mp * FRQ_T);
     float* ov = cv.take<float>(mp * FRQ_T);
+    if (use_gemv(w, m)) {  // the outputs in one pass, the same order
+        HIPCHK(launch_quant(d_a, m, w.k, w.kp, a8, sa, oi, ov, c->err, c->stream), "launch quant");
+        HIPCHK(launch_rows_i8(w, m, a8, sa, oi, ov, d_out, nullptr, c->stream), "launch rows_i8");
+        return FRQ_OK;
+    }
     void* gws = cv.take<char>(gemm_ws_bytes(m, w.kp, w.np));
     int32_t* acc = reinterpret_cast<int32_t*>((char*)c->ws + base);
     HIPCHK(launch_quant(d_a, m, w.k, w.kp, a8, sa, oi, ov, c->err, c->stream, mp), "launch quant");
@@ -649,11 +658,7 @@ int frq_mm_i8_q_dev(frq_ctx* c, const frq_w* wh, const int8_t* d_a8, const float
         return FRQ_OK;
     }
     if (use_gemv(w, m)) {
-        if (m == 1)
-            HIPCHK(launch_gemv_i8(w, m, d_a8, d_sa, d_oidx, d_oval, d_out, nullptr, c->stream), "launch gemv_i8");
-        else
-            HIPCHK(launch_skinny_i8(w, m, d_a8, d_sa, d_oidx, d_oval, d_out, nullptr, c->stream),
-                   "launch skinny_i8");
+        HIPCHK(launch_rows_i8(w, m, d_a8, d_sa, d_oidx, d_oval, d_out, nullptr, c->stream), "launch rows_i8");
         return FRQ_OK;
     }
     // the MFMA GEMM reads round_up(m, 128) rows of a8 in the blocked layout

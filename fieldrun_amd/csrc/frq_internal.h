@@ -479,6 +479,12 @@ __host__ __device__ inline size_t gated_col(size_t c, size_t hr) { return hr ? 2
 hipError_t launch_skinny_i8(const Weight& w, size_t m, const int8_t* a8, const float* sa,
                             const uint32_t* oidx, const float* oval, float* out, int32_t* acc,
                             hipStream_t s);
+// The same order for any m (a wave a 16-row tile): the middling batches that
+// mid_i8_ok picks.
+bool mid_i8_ok(const Weight& w, size_t m);
+hipError_t launch_mid_i8(const Weight& w, size_t m, const int8_t* a8, const float* sa,
+                         const uint32_t* oidx, const float* oval, float* out, int32_t* acc,
+                         hipStream_t s);
 // (valid rows of an (R, kp) row-major int8 matrix, pitch) -> blocked
 // (blk_off, R rows); rows >= valid become zero.
 hipError_t launch_blockify(const int8_t* src, size_t valid, size_t R, size_t kp,

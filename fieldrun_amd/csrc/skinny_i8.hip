@@ -120,6 +120,110 @@ __global__ __launch_bounds__(64 * KS) void skinny_i8_kernel(
     }
 }
 
+// 17 .. a few hundred rows, in the same order: a wave owns 16 token rows x CB
+// column blocks over all of K (A and B operands straight from a8 and wblk, U
+// k-blocks in flight; the four waves of a workgroup share the columns, so the
+// weights come to them from L1) and forms its outputs itself: the outliers'
+// weight bytes (16 rows x 32 channels x 16 CB columns from wkn, requested
+// before the k loop) wait in the wave's LDS and each lane adds the 32 terms
+// of its outputs in order.  No second pass over the sums, no barrier.  Bound
+// by the correction's three VALU instructions a term and, at long K, by L1
+// (1 KB + CB KB an MFMA pair).
+template <int CB>
+__global__ __launch_bounds__(256) void mid_i8_kernel(
+    const int8_t* __restrict__ Wb, const int8_t* __restrict__ Wkn, const float* __restrict__ scale, int N, int Np,
+    int Kp, const int8_t* __restrict__ a8, int M, const float* __restrict__ sa, const uint32_t* __restrict__ oidx,
+    const float* __restrict__ oval, int t, float* __restrict__ out, int32_t* __restrict__ acc_dbg) {
+    constexpr int TC = 16 * CB, RS = FRQ_T * TC + 16;  // RS: bytes a token's gathered rows (+16: other banks)
+    __shared__ __attribute__((aligned(16))) int8_t gat_[4][16 * RS];
+    __shared__ __attribute__((aligned(16))) float ovs_[4][16 * FRQ_T];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = ((int)blockIdx.y * 4 + wave) * 16, jb0 = blockIdx.x * CB, j0 = jb0 * 16;
+    if (m0 >= M) return;  // whole waves, no barrier below
+    int8_t* gat = gat_[wave];
+    float* ovs = ovs_[wave];
+    // the outlier gathers: pair p = (token p / 32, outlier p % 32)
+    v4i gv[8][CB];
+    float ovv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int p = lane + 64 * u, i = m0 + p / FRQ_T;
+        const bool ok = i < M && p % FRQ_T < t;
+        const size_t at = (size_t)(ok ? i : 0) * FRQ_T + p % FRQ_T;
+        const uint32_t ch = ok ? min(oidx[at], (uint32_t)(Kp - 1)) : 0u;
+        ovv[u] = ok ? oval[at] : 0.0f;
+#pragma unroll
+        for (int c = 0; c < CB; ++c) gv[u][c] = *reinterpret_cast<const v4i*>(Wkn + (size_t)ch * Np + j0 + 16 * c);
+    }
+    // lane 16 g + r: token row r (the last row past M), k-bytes 16 g ..
+    const int nkb = Kp / 64;
+    const int8_t* ap = a8 + (size_t)min(m0 + (lane & 15), M - 1) * Kp + 16 * (lane >> 4);
+    const int8_t* wp = Wb + (size_t)jb0 * 1024 + lane * 16;
+    const size_t kstride = (size_t)(Np / 16) * 1024;
+    v4i acc[CB];
+#pragma unroll
+    for (int c = 0; c < CB; ++c) acc[c] = v4i{0, 0, 0, 0};
+    constexpr int U = 4;
+    v4i an[U], bn[U][CB];
+    auto load = [&](int u, int kb) {  // unconditional: past the end the last block again
+        const int k = min(kb, nkb - 1);
+        an[u] = *reinterpret_cast<const v4i*>(ap + (size_t)k * 64);
+#pragma unroll
+        for (int c = 0; c < CB; ++c) bn[u][c] = *reinterpret_cast<const v4i*>(wp + (size_t)k * kstride + (size_t)c * 1024);
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(u, u);
+    for (int kb = 0; kb < nkb; kb += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (kb + u < nkb) {
+#pragma unroll
+                for (int c = 0; c < CB; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(an[u], bn[u][c], acc[c], 0, 0, 0);
+            }
+            load(u, kb + u + U);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int p = lane + 64 * u;
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+            *reinterpret_cast<v4i*>(gat + (p / FRQ_T) * RS + (p % FRQ_T) * TC + 16 * c) = gv[u][c];
+        ovs[p] = ovv[u];
+    }
+    wave_sync();
+    // lane l: tokens 4 (l / 16) + e, column l % 16 of each block
+    const int i0 = 4 * (lane >> 4);
+    float corr[4][CB];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) corr[e][c] = -0.0f;
+    for (int q = 0; q < t; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float ov = ovs[(i0 + e) * FRQ_T + q];
+#pragma unroll
+            for (int c = 0; c < CB; ++c)
+                corr[e][c] = corr[e][c] + ov * (float)gat[(i0 + e) * RS + q * TC + 16 * c + (lane & 15)];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int i = m0 + i0 + e;
+        if (i >= M) continue;
+        const float s = sa[i];
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            const int j = j0 + 16 * c + (lane & 15);
+            if (j >= N) continue;
+            out[(size_t)i * N + j] = scale[j] * (s * (float)acc[c][e] + corr[e][c]);
+            if (acc_dbg) acc_dbg[(size_t)i * N + j] = acc[c][e];
+        }
+    }
+}
+
 template <int CB, int KS>
 hipError_t launch_s(const Weight& w, size_t m, const int8_t* a8, const float* sa,
                     const uint32_t* oidx, const float* oval, float* out, int32_t* acc, hipStream_t s) {
@@ -130,7 +234,41 @@ hipError_t launch_s(const Weight& w, size_t m, const int8_t* a8, const float* sa
     return hipGetLastError();
 }
 
+template <int CB>
+hipError_t launch_m(const Weight& w, size_t m, const int8_t* a8, const float* sa, const uint32_t* oidx,
+                    const float* oval, float* out, int32_t* acc, hipStream_t s) {
+    const int t = (int)(w.k < FRQ_T ? w.k : FRQ_T);
+    const dim3 grid((unsigned)((w.n + 16 * CB - 1) / (16 * CB)), (unsigned)((m + 63) / 64));
+    mid_i8_kernel<CB><<<grid, dim3(256), 0, s>>>(w.wblk, w.wkn, w.scale, (int)w.n, (int)w.np, (int)w.kp, a8, (int)m,
+                                                 sa, oidx, oval, t, out, acc);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+// A 16 x 16 tile costs about 3.2 ns + 1.9 ps a k over the whole card
+// (measured for K 512 .. 14336, N 512 .. 30000, M 20 .. 512), the MFMA GEMM
+// with its correction 33 us at the least (the pre-pass, the split sums and the
+// epilogue), 60 .. 78 where K <= 2048 makes the outlier union dense: up to an
+// estimate of 30 us the tiles are faster (K=896 N=4864 M=129: 18 against 61;
+// K=4864 N=896: 18 against 42; K=4096 N=14336 M=48: 28 against 34, M=129
+// estimated at 90: 71 against 41).
+bool mid_i8_ok(const Weight& w, size_t m) {
+    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64) return false;
+    const double tiles = (double)((w.n + 15) / 16) * (double)((m + 15) / 16);
+    return tiles * (3.2 + 0.0019 * (double)w.kp) <= 30000.0;
+}
+
+hipError_t launch_mid_i8(const Weight& w, size_t m, const int8_t* a8, const float* sa, const uint32_t* oidx,
+                         const float* oval, float* out, int32_t* acc, hipStream_t s) {
+    // a8: m rows of pitch Kp; wblk / wkn padded to Np (a multiple of 256)
+    if (m < 1 || m > 65535 || !w.wblk || !w.wkn || w.kp % 64 || w.kp == 0) return hipErrorInvalidValue;
+    // two column blocks a wave from 1500 tiles on (us, one / two: K=896 N=4864
+    // M=48 11.8 / 11.4, M=129 19.9 / 17.9, M=512 55 / 41; K=4096 N=14336 M=20
+    // 31.7 / 21.1; K=2048 N=2048 M=129 12.3 / 15.5, M=256 20.0 / 15.9)
+    if ((w.n + 15) / 16 * ((m + 15) / 16) > 1500) return launch_m<2>(w, m, a8, sa, oidx, oval, out, acc, s);
+    return launch_m<1>(w, m, a8, sa, oidx, oval, out, acc, s);
+}
 
 hipError_t launch_skinny_i8(const Weight& w, size_t m, const int8_t* a8, const float* sa,
                             const uint32_t* oidx, const float* oval, float* out, int32_t* acc,

@@ -346,3 +346,20 @@ def test_i4_m1_bit_exact_avx2_order(ctx, n, k):
     ref = oracle.mm_i4(a, packed, s16.astype(np.float32), k, g)
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
     w.free()
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 896, 4864), (31, 37, 50), (32, 64, 17), (33, 1000, 3000), (64, 20, 33),
+                                   (65, 4864, 896), (129, 2048, 130), (200, 128, 129), (512, 512, 512), (48, 4096, 8000),
+                                   (20, 14336, 257), (300, 896, 1601)])
+def test_i8_middling_batches_bit_exact(ctx, m, k, n):
+    """17 .. a few hundred rows on the one-pass tiles (one and two column
+    blocks a wave, ragged M, N and K, K below the outlier count): sums and
+    outputs bit for bit against the oracle, also through frq_mm_exact_dev."""
+    a, wt, scale = case(m, k, n, 500 + m + k + n)
+    w = ctx.upload_i8(wt, scale)
+    out, acc, a8, sa, oi, ov = w.mm_debug(a)
+    ref, racc = oracle.mm_i8(a, wt, scale, with_acc=True)
+    assert np.array_equal(acc, racc)
+    check_quant(a, a8, sa, oi, ov)
+    assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(w.mm_exact(a).view(np.uint32), ref.view(np.uint32))
