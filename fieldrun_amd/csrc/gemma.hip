@@ -990,6 +990,8 @@ __global__ __launch_bounds__(GT) void gm_attn_tile_kernel(const float* __restric
 // st[kv][block][key][pair] (kpad keys a block) that the second launch turns
 // into exps in place.
 constexpr int PF_AP = 64, PF_KT = 128, PF_VK = 64, PF_NT = 256;
+constexpr int PF_PP = PF_AP + 16;  // p's LDS row: 16 pairs of four keys on all banks
+typedef float f4v __attribute__((ext_vector_type(4)));
 static_assert(MM_KC % PF_VK == 0, "a value chunk lies in one a.dot block");
 constexpr size_t PF_MIN_ROWS = 1024;  // shorter prompts take the one-launch kernels (more workgroups)
 constexpr size_t PF_MAX_BYTES = (size_t)2 << 30;  // score buffer cap (570 MB at configs[4]'s 2048 + 128)
@@ -1006,9 +1008,11 @@ __device__ __forceinline__ PfRow pf_row(int i, int cur, int m, int sliding, int 
 // 1. scores: workgroup (kv, block b), heaviest blocks first; the block's q
 // pairs in LDS, then its key tiles in order, each tile's 128 key rows in
 // LDS (rows HD + 4 floats apart) while the next tile's rows load into
-// registers; a lane 8 pairs x 4 keys (keys kg + 32u); writes the scaled
-// (capped) scores and each pair's max over every tile key its row sees.
-template <int RP, int RV, int HD>
+// registers; the products are v_mfma_f32_16x16x4 (an FMA chain in ascending
+// dim, a.dot's order for HD <= 256); writes the scaled (capped) scores and
+// each pair's max over every tile key its row sees.  Bound by the f32 MFMAs
+// and their operand reads (six 4-byte LDS reads for eight).
+template <int RP, int HD>
 __global__ __launch_bounds__(PF_NT) void gm_pf_scores_kernel(const float* __restrict__ qkv, int H, int KV,
                                                              const int* __restrict__ curp, int m,
                                                              const float* __restrict__ kc, float qscale, float cap,
@@ -1049,19 +1053,23 @@ __global__ __launch_bounds__(PF_NT) void gm_pf_scores_kernel(const float* __rest
         const int x = tid + u * PF_NT;
         *reinterpret_cast<float4*>(Qs + (x / H4) * HP + 4 * (x % H4)) = qv[u];
     }
-    const int kg = tid & 31, pg = tid >> 5;
+    // wave w: the tile's keys 32 w .. + 31 (two 16-key column tiles) against
+    // all 64 pairs (four row tiles); lane (h = lane / 16, i = lane % 16)
+    // feeds dims 4 s + h of row i of a tile and holds pairs 16 t + 4 h + v of
+    // key 16 u + i
+    const int lane = tid & 63, wave = tid >> 6, li = lane & 15, lh = lane >> 4;
+    __shared__ float wmax[PF_NT / 64][PF_AP];
     float* sb = st + ((size_t)kv * nrb + b) * (size_t)kpad * PF_AP;
-    // rows of this lane's pairs: keys [j0, nk) (nk 0 past m)
-    int rj0[8], rnk[8];
+    auto row_of = [&](int t, int v) {  // keys [j0, nk) of a pair's row (none past m)
+        PfRow rw = pf_row(r0 + (16 * t + 4 * lh + v) / RP, cur, m, sliding, window);
+        if (!rw.ok) rw.nk = 0;
+        return rw;
+    };
+    float mxl[4][4];
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        const PfRow rw = pf_row(r0 + (8 * pg + a) / RP, cur, m, sliding, window);
-        rj0[a] = rw.j0;
-        rnk[a] = rw.ok ? rw.nk : 0;
-    }
-    float mxl[8];
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int a = 0; a < 8; ++a) mxl[a] = -INFINITY;
+        for (int v = 0; v < 4; ++v) mxl[t][v] = -INFINITY;
     for (int c = 0; c < ntile; ++c) {
         __syncthreads();  // the previous tile is consumed
 #pragma unroll
@@ -1071,71 +1079,76 @@ __global__ __launch_bounds__(PF_NT) void gm_pf_scores_kernel(const float* __rest
         }
         __syncthreads();
         if (c + 1 < ntile) kload(c + 1);  // in flight during this tile
-        float acc[8][4];
+        f4v acc[4][2];
 #pragma unroll
-        for (int a = 0; a < 8; ++a)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) acc[a][u] = 0.0f;
-        const float* qb = Qs + (8 * pg) * HP;
-        const float* kb = Ks + kg * HP;
-#pragma unroll 2
+            for (int u = 0; u < 2; ++u) acc[t][u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+        const float* qb = Qs + li * HP + lh;
+        const float* kb = Ks + (32 * wave + li) * HP + lh;
+#pragma unroll 8
         for (int sd = 0; sd < H4; ++sd) {
-            float4 q4[8], k4[4];
+            float q[4], k[2];
 #pragma unroll
-            for (int a = 0; a < 8; ++a)
-                if (a % RP < RV) q4[a] = *reinterpret_cast<const float4*>(qb + a * HP + 4 * sd);
+            for (int t = 0; t < 4; ++t) q[t] = qb[16 * t * HP + 4 * sd];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) k4[u] = *reinterpret_cast<const float4*>(kb + 32 * u * HP + 4 * sd);
+            for (int u = 0; u < 2; ++u) k[u] = kb[16 * u * HP + 4 * sd];
 #pragma unroll
-            for (int a = 0; a < 8; ++a)
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (a % RP >= RV) continue;  // a spare head: never leaves the kernel
-                    acc[a][u] = __builtin_fmaf(q4[a].x, k4[u].x, acc[a][u]);
-                    acc[a][u] = __builtin_fmaf(q4[a].y, k4[u].y, acc[a][u]);
-                    acc[a][u] = __builtin_fmaf(q4[a].z, k4[u].z, acc[a][u]);
-                    acc[a][u] = __builtin_fmaf(q4[a].w, k4[u].w, acc[a][u]);
-                }
+                for (int u = 0; u < 2; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[t], k[u], acc[t][u], 0, 0, 0);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = c * PF_KT + kg + 32 * u;
-            float sv[8];
+        for (int u = 0; u < 2; ++u) {
+            const int j = c * PF_KT + 32 * wave + 16 * u + li;
 #pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                float sj = div ? acc[a][u] / qscale : acc[a][u] * qscale;
-                if (cap > 0.0f) sj = cap * libm::frq_tanhf(sj / cap);
-                sv[a] = sj;
-                if (j >= rj0[a] && j < rnk[a]) mxl[a] = fmaxf(mxl[a], sj);
+            for (int t = 0; t < 4; ++t) {
+                float4 sv;
+                float* se = &sv.x;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float sj = div ? acc[t][u][v] / qscale : acc[t][u][v] * qscale;
+                    if (cap > 0.0f) sj = cap * libm::frq_tanhf(sj / cap);
+                    se[v] = sj;
+                    const PfRow rw = row_of(t, v);
+                    if (j >= rw.j0 && j < rw.nk) mxl[t][v] = fmaxf(mxl[t][v], sj);
+                }
+                *reinterpret_cast<float4*>(sb + (size_t)j * PF_AP + 16 * t + 4 * lh) = sv;
             }
-            float4* dst = reinterpret_cast<float4*>(sb + (size_t)j * PF_AP + 8 * pg);
-            dst[0] = make_float4(sv[0], sv[1], sv[2], sv[3]);
-            dst[1] = make_float4(sv[4], sv[5], sv[6], sv[7]);
         }
     }
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        float v = mxl[a];
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int off = 16; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-        if (kg == 0) pmax[((size_t)kv * nrb + b) * PF_AP + 8 * pg + a] = v;
+        for (int v = 0; v < 4; ++v) {
+            float x = mxl[t][v];
+#pragma unroll
+            for (int off = 8; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off, 64));
+            if (li == 0) wmax[wave][16 * t + 4 * lh + v] = x;
+        }
+    __syncthreads();
+    if (tid < PF_AP) {
+        float x = wmax[0][tid];
+#pragma unroll
+        for (int w = 1; w < PF_NT / 64; ++w) x = fmaxf(x, wmax[w][tid]);
+        pmax[((size_t)kv * nrb + b) * PF_AP + tid] = x;
     }
 }
 
 // 2. workgroup (kv, block b), heaviest first: the pairs' maxes (one per
 // pair from the first launch); per key tile the exps (branch-free) into LDS
 // and, in place of the scores, into st, then wave 0 adds them in key order
-// (a lane a pair); then the value chains, a lane 8 pairs x 4 dims, over
-// 64-key chunks of p = e / sum and the value rows staged in LDS, the next
-// chunk loading into registers meanwhile (chunks every row of the block
-// sees entirely run without per-key tests).
-template <int RP, int RV, int HD>
-__global__ __launch_bounds__(PF_NT) void gm_pf_values_kernel(int H, int KV, const int* __restrict__ curp, int m,
+// (a lane a pair); then the value chains on v_mfma_f32_16x16x4, ascending
+// keys from +0, over 64-key chunks of p = e / sum and the value rows staged
+// in LDS, the next chunk loading into registers meanwhile.
+template <int RP, int HD>
+__global__ __launch_bounds__(PF_NT, 2) void gm_pf_values_kernel(int H, int KV, const int* __restrict__ curp, int m,
                                                              const float* __restrict__ vc, int sliding, int window,
                                                              int nrb, int kpad, float* __restrict__ st,
                                                              const float* __restrict__ pmax,
                                                              float* __restrict__ att) {
-    constexpr int RB = PF_AP / RP, HP = HD + 4, H4 = HD / 4;
+    constexpr int RB = PF_AP / RP, H4 = HD / 4;
     constexpr int PN = PF_VK * PF_AP / PF_NT, VN = (PF_VK * H4 + PF_NT - 1) / PF_NT;
     extern __shared__ float4 lds4[];
     __shared__ float mx[PF_AP], sums[PF_AP];
@@ -1195,29 +1208,21 @@ __global__ __launch_bounds__(PF_NT) void gm_pf_values_kernel(int H, int KV, cons
     }
     if (tid < PF_AP) sums[tid] = sm;
     __syncthreads();
-    // values
-    float* Ps = reinterpret_cast<float*>(lds4);  // [PF_VK][PF_AP]
-    float* Vs = Ps + PF_VK * PF_AP;              // [PF_VK][HP]
-    const int pg = tid >> 5, dg = tid & 31;
-    const bool lane_on = dg < H4;
-    int rj0[8], rnk[8];
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        const PfRow rw = pf_row(r0 + (8 * pg + a) / RP, cur, m, sliding, window);
-        rj0[a] = rw.j0;
-        rnk[a] = rw.ok ? rw.nk : 0;
-    }
-    // keys every row of the block sees: [j0 of the last row, nk of the first)
-    const PfRow rfirst = pf_row(r0, cur, m, sliding, window);
-    const PfRow rlast = pf_row(min(r0 + RB, m) - 1, cur, m, sliding, window);
+    // values: the block's 64 pairs (four row tiles) x the wave's NTV tiles of
+    // 16 dims; a key outside a pair's row has p = 0 (e = 0), an exact zero term
+    float* Ps = reinterpret_cast<float*>(lds4);  // [PF_VK][PF_PP]
+    float* Vs = Ps + PF_VK * PF_PP;              // [PF_VK][VP]
+    constexpr int NTV = HD >= 64 ? HD / 64 : 1, VP = HD + 16;
+    const int lane = tid & 63, wave = tid >> 6, li = lane & 15, lh = lane >> 4;
+    const bool wave_on = 16 * NTV * wave < HD;
     const float rsum = sums[pq];
     // a.dot's order: each MM_KC-key block (chunks from 0, MM_KC a multiple
     // of PF_VK) chained from +0 in acc, the blocks added in order into tot
-    float acc[8][4], tot[8][4];
+    f4v acc[4][NTV], tot[4][NTV];
 #pragma unroll
-    for (int a = 0; a < 8; ++a)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) acc[a][d] = tot[a][d] = 0.0f;
+        for (int u = 0; u < NTV; ++u) acc[t][u] = tot[t][u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
     const int nvc = (kend + PF_VK - 1) / PF_VK;
     float pn[PN];
     float4 vn[VN];
@@ -1241,97 +1246,87 @@ __global__ __launch_bounds__(PF_NT) void gm_pf_values_kernel(int H, int KV, cons
         const int jc = c * PF_VK;
         __syncthreads();  // the previous chunk is consumed
 #pragma unroll
-        for (int u = 0; u < PN; ++u) Ps[tid + u * PF_NT] = pn[u] / rsum;  // pair tid % 64 throughout
+        for (int u = 0; u < PN; ++u) {  // pair tid % 64 throughout
+            const int x = tid + u * PF_NT;
+            Ps[x / PF_AP * PF_PP + x % PF_AP] = pn[u] / rsum;
+        }
 #pragma unroll
         for (int u = 0; u < VN; ++u) {
             const int x = tid + u * PF_NT;
-            if (x < PF_VK * H4) *reinterpret_cast<float4*>(Vs + (x / H4) * HP + 4 * (x % H4)) = vn[u];
+            if (x < PF_VK * H4) *reinterpret_cast<float4*>(Vs + (x / H4) * VP + 4 * (x % H4)) = vn[u];
         }
         __syncthreads();
         if (c + 1 < nvc) cload(c + 1);
         if (jc > 0 && jc % MM_KC == 0) {
 #pragma unroll
-            for (int a = 0; a < 8; ++a)
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    tot[a][d] = tot[a][d] + acc[a][d];
-                    acc[a][d] = 0.0f;
-                }
-        }
-        const bool full = jc >= rlast.j0 && jc + PF_VK <= rfirst.nk;
-        if (lane_on && full) {
-            for (int t = 0; t < PF_VK; ++t) {
-                const float4 pa = *reinterpret_cast<const float4*>(Ps + t * PF_AP + 8 * pg);
-                const float4 pb = *reinterpret_cast<const float4*>(Ps + t * PF_AP + 8 * pg + 4);
-                const float4 v = *reinterpret_cast<const float4*>(Vs + t * HP + 4 * dg);
-                const float pv[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
-                const float vv[4] = {v.x, v.y, v.z, v.w};
+                for (int u = 0; u < NTV; ++u)
 #pragma unroll
-                for (int a = 0; a < 8; ++a) {
-                    if (a % RP >= RV) continue;
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) acc[a][d] = __builtin_fmaf(pv[a], vv[d], acc[a][d]);
-                }
-            }
-        } else if (lane_on) {
-            for (int t = 0; t < PF_VK; ++t) {
-                const int j = jc + t;
-                const float4 pa = *reinterpret_cast<const float4*>(Ps + t * PF_AP + 8 * pg);
-                const float4 pb = *reinterpret_cast<const float4*>(Ps + t * PF_AP + 8 * pg + 4);
-                const float4 v = *reinterpret_cast<const float4*>(Vs + t * HP + 4 * dg);
-                const float pv[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int a = 0; a < 8; ++a) {
-                    if (a % RP >= RV) continue;
-                    const bool on = j >= rj0[a] && j < rnk[a];
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const float n = __builtin_fmaf(pv[a], vv[d], acc[a][d]);
-                        acc[a][d] = on ? n : acc[a][d];
+                    for (int v = 0; v < 4; ++v) {
+                        tot[t][u][v] = tot[t][u][v] + acc[t][u][v];
+                        acc[t][u][v] = 0.0f;
                     }
-                }
+        }
+        if (wave_on) {
+            const float* pb = Ps + lh * PF_PP + li;
+            const float* vb = Vs + lh * VP + 16 * NTV * wave + li;
+#pragma unroll 8
+            for (int sk = 0; sk < PF_VK / 4; ++sk) {
+                float pr[4], vv[NTV];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) pr[t] = pb[4 * sk * PF_PP + 16 * t];
+#pragma unroll
+                for (int u = 0; u < NTV; ++u) vv[u] = vb[4 * sk * VP + 16 * u];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int u = 0; u < NTV; ++u)
+                        acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[t], vv[u], acc[t][u], 0, 0, 0);
             }
         }
     }
-    if (lane_on) {
+    if (wave_on) {
 #pragma unroll
-        for (int a = 0; a < 8; ++a) {
-            const int pp = 8 * pg + a, h = pp % RP, i = r0 + pp / RP;
-            if (h < R && i < m)
-                *reinterpret_cast<float4*>(att + (size_t)i * H * HD + (size_t)(kv * R + h) * HD + 4 * dg) =
-                    make_float4(tot[a][0] + acc[a][0], tot[a][1] + acc[a][1], tot[a][2] + acc[a][2],
-                                tot[a][3] + acc[a][3]);
-        }
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int pp = 16 * t + 4 * lh + v, h = pp % RP, i = r0 + pp / RP;
+                if (h >= R || i >= m) continue;
+#pragma unroll
+                for (int u = 0; u < NTV; ++u)
+                    att[(size_t)i * H * HD + (size_t)(kv * R + h) * HD + 16 * (NTV * wave + u) + li] =
+                        tot[t][u][v] + acc[t][u][v];
+            }
     }
 }
 
 // LDS and scratch of the two-launch prefill attention
 inline size_t pf_scores_lds(int hd) { return (size_t)(PF_AP + PF_KT) * (hd + 4) * sizeof(float); }
 inline size_t pf_values_lds(int hd) {
-    return std::max((size_t)PF_KT * PF_AP, (size_t)PF_VK * PF_AP + (size_t)PF_VK * (hd + 4)) * sizeof(float);
+    return std::max((size_t)PF_KT * PF_AP, (size_t)PF_VK * PF_PP + (size_t)PF_VK * (hd + 16)) * sizeof(float);
 }
 inline size_t pf_kpad(size_t npos) { return (npos + PF_KT - 1) / PF_KT * PF_KT; }
 
-template <int RP, int RV, int HD>
+template <int RP, int HD>
 hipError_t launch_pf_t(const float* qkv, int H, int KV, const int* cur, int m, const float* kc, const float* vc,
                        float qscale, float cap, int sl, int win, int nrb, int nkt, int kpad, float* st, float* pmx,
                        float* att, int div, hipStream_t s) {
     const size_t l1 = pf_scores_lds(HD), l2 = pf_values_lds(HD);
     static bool attr = false;  // per process; the attribute is per function
     if (!attr) {
-        if (hipError_t e = hipFuncSetAttribute((const void*)gm_pf_scores_kernel<RP, RV, HD>,
+        if (hipError_t e = hipFuncSetAttribute((const void*)gm_pf_scores_kernel<RP, HD>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)l1))
             return e;
-        if (hipError_t e = hipFuncSetAttribute((const void*)gm_pf_values_kernel<RP, RV, HD>,
+        if (hipError_t e = hipFuncSetAttribute((const void*)gm_pf_values_kernel<RP, HD>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)l2))
             return e;
         attr = true;
     }
-    gm_pf_scores_kernel<RP, RV, HD><<<dim3((unsigned)(KV * nrb)), dim3(PF_NT), l1, s>>>(
+    gm_pf_scores_kernel<RP, HD><<<dim3((unsigned)(KV * nrb)), dim3(PF_NT), l1, s>>>(
         qkv, H, KV, cur, m, kc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, div);
     if (hipError_t e = hipGetLastError()) return e;
-    gm_pf_values_kernel<RP, RV, HD><<<dim3((unsigned)(KV * nrb)), dim3(PF_NT), l2, s>>>(H, KV, cur, m, vc, sl, win, nrb,
+    gm_pf_values_kernel<RP, HD><<<dim3((unsigned)(KV * nrb)), dim3(PF_NT), l2, s>>>(H, KV, cur, m, vc, sl, win, nrb,
                                                                                  kpad, st, pmx, att);
     return hipGetLastError();
 }
@@ -1340,13 +1335,9 @@ template <int HD>
 hipError_t launch_pf_h(int rp, const float* qkv, int H, int KV, const int* cur, int m, const float* kc,
                        const float* vc, float qscale, float cap, int sl, int win, int nrb, int nkt, int kpad, float* st,
                        float* pmx, float* att, int div, hipStream_t s) {
-    // RV: the heads the FMAs run on (the spare ones of RP > R only where
-    // R == 7, the Qwen2.5-7B group; elsewhere they run on zero q)
-    const int R = H / KV;
-    if (rp == 2) return launch_pf_t<2, 2, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
-    if (rp == 4) return launch_pf_t<4, 4, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
-    if (R == 7) return launch_pf_t<8, 7, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
-    return launch_pf_t<8, 8, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
+    if (rp == 2) return launch_pf_t<2, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
+    if (rp == 4) return launch_pf_t<4, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
+    return launch_pf_t<8, HD>(qkv, H, KV, cur, m, kc, vc, qscale, cap, sl, win, nrb, nkt, kpad, st, pmx, att, div, s);
 }
 
 hipError_t launch_pf_attention(int rp, int hd, const float* qkv, int H, int KV, const int* cur, int m,
