@@ -1210,11 +1210,16 @@ __global__ __launch_bounds__(PF_NT, 2) void gm_pf_values_kernel(int H, int KV, c
     __syncthreads();
     // values: the block's 64 pairs (four row tiles) x the wave's NTV tiles of
     // 16 dims; a key outside a pair's row has p = 0 (e = 0), an exact zero term
+    // unless its value is an infinity or NaN: a chunk that holds one of these
+    // and that not every row of the block sees whole is walked key by key
     float* Ps = reinterpret_cast<float*>(lds4);  // [PF_VK][PF_PP]
     float* Vs = Ps + PF_VK * PF_PP;              // [PF_VK][VP]
     constexpr int NTV = HD >= 64 ? HD / 64 : 1, VP = HD + 16;
     const int lane = tid & 63, wave = tid >> 6, li = lane & 15, lh = lane >> 4;
     const bool wave_on = 16 * NTV * wave < HD;
+    // keys every row of the block sees: [j0 of the last row, nk of the first)
+    const int seen0 = pf_row(min(r0 + RB, m) - 1, cur, m, sliding, window).j0;
+    const int seen1 = pf_row(r0, cur, m, sliding, window).nk;
     const float rsum = sums[pq];
     // a.dot's order: each MM_KC-key block (chunks from 0, MM_KC a multiple
     // of PF_VK) chained from +0 in acc, the blocks added in order into tot
@@ -1255,7 +1260,16 @@ __global__ __launch_bounds__(PF_NT, 2) void gm_pf_values_kernel(int H, int KV, c
             const int x = tid + u * PF_NT;
             if (x < PF_VK * H4) *reinterpret_cast<float4*>(Vs + (x / H4) * VP + 4 * (x % H4)) = vn[u];
         }
-        __syncthreads();
+        bool by_key = false;  // uniform over the workgroup
+        if (jc >= seen0 && jc + PF_VK <= seen1) {
+            __syncthreads();
+        } else {
+            float z = 0.0f;  // NaN with any value that is not finite
+#pragma unroll
+            for (int u = 0; u < VN; ++u)
+                z += 0.0f * vn[u].x + 0.0f * vn[u].y + (0.0f * vn[u].z + 0.0f * vn[u].w);
+            by_key = __syncthreads_or(z != z);
+        }
         if (c + 1 < nvc) cload(c + 1);
         if (jc > 0 && jc % MM_KC == 0) {
 #pragma unroll
@@ -1268,7 +1282,21 @@ __global__ __launch_bounds__(PF_NT, 2) void gm_pf_values_kernel(int H, int KV, c
                         acc[t][u][v] = 0.0f;
                     }
         }
-        if (wave_on) {
+        if (wave_on && by_key) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int pp = 16 * t + 4 * lh + v;
+                    const PfRow rw = pf_row(r0 + pp / RP, cur, m, sliding, window);
+                    const int ka = max(rw.j0 - jc, 0), kb = rw.ok ? min(rw.nk - jc, PF_VK) : 0;
+                    for (int k = ka; k < kb; ++k)
+#pragma unroll
+                        for (int u = 0; u < NTV; ++u)
+                            acc[t][u][v] = __builtin_fmaf(Ps[k * PF_PP + pp], Vs[k * VP + 16 * (NTV * wave + u) + li],
+                                                          acc[t][u][v]);
+                }
+        } else if (wave_on) {
             const float* pb = Ps + lh * PF_PP + li;
             const float* vb = Vs + lh * VP + 16 * NTV * wave + li;
 #pragma unroll 8

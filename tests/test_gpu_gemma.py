@@ -4,6 +4,8 @@ tokens and logits bit for bit, for int4 / int8 / q4a linears, the f32 and
 int8 caches, prompts of 1, 5, 20 rows, the captured-graph decode equal to
 the eager one, the sliding window (a prompt past 4096 positions), and
 configs[2] (Gemma-2-2b, int4) at full size on a short sample."""
+import json
+
 import numpy as np
 import pytest
 
@@ -104,6 +106,35 @@ def test_config2_gemma2_2b_int4(ctx, tmp_path):
     rt, rlg = ref.generate(prompt, 4, with_logits=True)
     assert np.array_equal(toks, rt)
     assert same_bits(lg, rlg), first_diff(lg, rlg)
+    g.free()
+    b.close()
+
+
+def test_gemma_prefill_ignores_non_finite_values_behind_window(ctx, tmp_path):
+    """A token whose layer-0 value row is not finite, more than the window
+    behind the prompt's last row, takes no part in that row's attention
+    (prompts of 1024 rows and more): the same logits as with a finite token
+    there.  That token's embedding is 3e38 in one channel: infinite once
+    scaled, NaN after the norm, and a logit that the final cap bounds."""
+    stem = str(tmp_path / "n")
+    synth.write_gemma2_bundle(stem, 18, n_layer=1, n_head=2, n_kv=1, hd=32, d=64, ffn=64, vocab=300, std=0.1,
+                              embed="f32")
+    bad, ok = 7, 8
+    at = next(e["offset"] for e in json.load(open(stem + ".fieldrun.json"))["arrays"] if e["name"] == "embed")
+    blob = np.memmap(stem + ".fieldrun.bin", np.uint8, "r+")
+    embed = blob[at:at + 300 * 64 * 4].view(np.float32).reshape(300, 64)
+    embed[bad] = 0.0
+    embed[bad, 3] = 3e38
+    blob.flush()
+    prompt = synth.gpt2_prompt(4200, 300, 19)
+    prompt[prompt == bad] = ok
+    b = fa.Bundle(stem, ctx)
+    g = fa.Gemma(b)
+    toks, lg = g.generate(prompt, 1, with_logits=True)
+    prompt[5] = bad
+    tb, lgb = g.generate(prompt, 1, with_logits=True)
+    assert np.isfinite(lg).all() and np.array_equal(tb, toks)
+    assert same_bits(lgb, lg)
     g.free()
     b.close()
 
