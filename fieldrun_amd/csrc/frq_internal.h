@@ -553,7 +553,7 @@ hipError_t launch_pack_m1_any(bool q4a, const uint8_t* packed, size_t pitch, con
 hipError_t launch_i4_exact(const Weight& w, size_t m, const float* a, float* out, hipStream_t s);
 // m rows each in the M == 1 order (i4_dot_avx2), weights read once.
 // Batched decode rows (m independent rows, each in the M == 1 order):
-// i4_rows_a4_ok says whether the weight takes the broadcast kernel, which
+// i4_rows_a4_ok says whether the weight takes the batched kernel, which
 // reads its <= 16 rows in the a4 layout (launch_rows_to_a4: the rows
 // interleaved by k-quads, i4_a4_floats(K) floats); launch_i4_m1_rows takes
 // row-major rows and a4 scratch (or NULL: one M == 1 launch a row).

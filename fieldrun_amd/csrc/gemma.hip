@@ -2057,7 +2057,7 @@ int gm_mm(frq_ctx* c, const frq_w* wh, const float* in, size_t m, float* outp) {
 // The linears of a batch step: m rows, each its own sequence's decode row,
 // so each row in the M == 1 order of its dtype (int8: the multi-row path is
 // bit-identical to M == 1 up to 16 rows; int4: i4_dot_avx2's order for every
-// row, a4 the broadcast kernel's staging of i4_a4_floats(K) floats; q4a: one
+// row, a4 the batched kernel's staging of i4_a4_floats(K) floats; q4a: one
 // M == 1 call a row).
 int gm_mm_rows(frq_ctx* c, const frq_w* wh, const float* in, size_t m, float* outp, float* a4) {
     const Weight& w = *weight_of(wh);

@@ -33,7 +33,7 @@
 // and invalidate the whole L2.
 // Other shapes run i4_gemv_generic (M == 1, bit-identical to i4_dot_avx2)
 // or, M > 1 in the exact order, the f32 matrix cores (mm_f32.hip).  Up to 16
-// independent M == 1 rows (a batched decode) run i4_rows_dpp.
+// independent M == 1 rows (a batched decode) run i4_rows_mfma.
 #include "frq_internal.h"
 
 namespace frq {
@@ -330,47 +330,11 @@ __global__ __launch_bounds__(NT) void i4_m1_stream(const uint8_t* __restrict__ p
     for (int rr = tid; rr < nr; rr += NT) out[r0 + rr] = lds_seq_sum(terms + rr * ngp, ng, 0.0f);
 }
 
-// 16 FMAs of one weight register v of a 32-unit into lane chains
-// l[4 v .. 4 v + 3]: v_fmac_f32_dpp with row_newbcast:n gives each token
-// lane of a 16-lane DPP row the weight held by lane n of that row.  Lane n
-// holds element e = 8 (n & 3) + (n >> 2) + 4 v, which is nibble
-// (n >> 2) + 4 v of word n & 3 (chain q = e & 7, chunk c = e >> 3), and its
-// product takes av[e]; the FMAs go c-major so each chain advances in chunk
-// order.  START begins the chains: chunk 0 is a v_mul_f32_dpp, which
-// differs from fma(w, a, +0) only in giving -0 for a -0 product; a chain
-// is exact otherwise, the lane sums of i4_dot_avx2 then differ at most in
-// the sign of a zero, and so does a group term, which the running sum from
-// +0 absorbs (+0 + -0 == +0): the row sums are bit-identical.  The s_nop
-// gives the two wait states a DPP read needs after the VALU write of w,
-// which the compiler does not see inside the asm.
-#define FRQ_DPPF(op, acc, n, src) #op "_f32_dpp %" #acc ", %4, %" #src " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
-#define FRQ_DPP_C0(op) FRQ_DPPF(op, 0, 0, 5) FRQ_DPPF(op, 1, 4, 9) FRQ_DPPF(op, 2, 8, 13) FRQ_DPPF(op, 3, 12, 17)
-#define FRQ_DPP_C123                                                                                          \
-    FRQ_DPPF(v_fmac, 0, 1, 6) FRQ_DPPF(v_fmac, 1, 5, 10) FRQ_DPPF(v_fmac, 2, 9, 14) FRQ_DPPF(v_fmac, 3, 13, 18) \
-    FRQ_DPPF(v_fmac, 0, 2, 7) FRQ_DPPF(v_fmac, 1, 6, 11) FRQ_DPPF(v_fmac, 2, 10, 15)                            \
-    FRQ_DPPF(v_fmac, 3, 14, 19) FRQ_DPPF(v_fmac, 0, 3, 8) FRQ_DPPF(v_fmac, 1, 7, 12)                            \
-    FRQ_DPPF(v_fmac, 2, 11, 16) FRQ_DPPF(v_fmac, 3, 15, 20)
-#define FRQ_DPP_OPS(V)                                                                              \
-    : "+v"(l[4 * V]), "+v"(l[4 * V + 1]), "+v"(l[4 * V + 2]), "+v"(l[4 * V + 3])                    \
-    : "v"(w), "v"(av[4 * V]), "v"(av[8 + 4 * V]), "v"(av[16 + 4 * V]), "v"(av[24 + 4 * V]),         \
-      "v"(av[1 + 4 * V]), "v"(av[9 + 4 * V]), "v"(av[17 + 4 * V]), "v"(av[25 + 4 * V]),             \
-      "v"(av[2 + 4 * V]), "v"(av[10 + 4 * V]), "v"(av[18 + 4 * V]), "v"(av[26 + 4 * V]),            \
-      "v"(av[3 + 4 * V]), "v"(av[11 + 4 * V]), "v"(av[19 + 4 * V]), "v"(av[27 + 4 * V])
-template <int V, bool START>
-__device__ __forceinline__ void dpp_fma16(float (&l)[8], float w, const float (&av)[32]) {
-    if constexpr (START)
-        asm("s_nop 1\n\t" FRQ_DPP_C0(v_mul) FRQ_DPP_C123 FRQ_DPP_OPS(V));
-    else
-        asm("s_nop 1\n\t" FRQ_DPP_C0(v_fmac) FRQ_DPP_C123 FRQ_DPP_OPS(V));
-}
-#undef FRQ_DPP_OPS
-#undef FRQ_DPP_C123
-#undef FRQ_DPP_C0
-#undef FRQ_DPPF
+constexpr int ROWS_GW = 4;  // groups a wave of i4_rows_mfma takes a round, at most
 
-// The activation layout of i4_rows_dpp: the 16 token rows interleaved by
+// The activation layout of i4_rows_mfma: the 16 token rows interleaved by
 // k-quads, a4[64 (k / 4) + 4 t + k % 4] = a[t][k] (rows t >= M zero), so
-// that the 16 token lanes of a DPP row read 256 contiguous bytes a load.
+// that 16 token lanes read 256 contiguous bytes a load.
 __global__ void rows_to_a4_kernel(const float* __restrict__ a, int M, int K, float* __restrict__ a4) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;  // float4 i of a4: k-quad i / 16, token i % 16
     const int kq = i >> 4, t = i & 15;
@@ -380,153 +344,118 @@ __global__ void rows_to_a4_kernel(const float* __restrict__ a, int M, int K, flo
     reinterpret_cast<float4*>(a4)[i] = v;
 }
 
-// M independent rows (M <= 16), each in the M == 1 order (i4_dot_avx2),
-// with the weights broadcast across tokens: lane 16 d + t of a wave is token
-// t in DPP row d, and the workgroup's ND = 4 NW DPP rows D = 4 wave + d take
-// a slice of 2 ND groups in two rounds (groups 2 ND s + ND i + D, i = 0, 1).
-// A lane holds its token's 32 activations of the current 32-unit (read from
-// the a4 layout) and, for each of the workgroup's R weight rows, the packed
-// word t & 3 of the unit, whose nibbles t >> 2 and 4 + (t >> 2) become its
-// two f32 weight registers (dpp_fma16): each activation register serves R
-// rows and each weight register 16 tokens.  A group's term scale * gsum goes
-// to LDS (+0 for the groups past the end, which the running sum absorbs
-// exactly: it is never -0); after the slice's one barrier the lane of (row,
-// token) adds the slice's 2 ND terms to its running sum in group order (two
-// term buffers, so the next slice's writes never meet this slice's reads).
-// Activations and scales are loaded one step ahead, weights two.  Needs
-// K % (32 G4) == 0 and a matrix under 4 GB (32-bit offsets from each row's
-// base).
-template <int G4, int R, int NW>
-__global__ __launch_bounds__(64 * NW) void i4_rows_dpp(const uint8_t* __restrict__ packed,
-                                                       const uint16_t* __restrict__ scale, int N, int K,
+// M independent rows (M <= 16), each in the M == 1 order (i4_dot_avx2), on
+// the f32 matrix cores: v_mfma_f32_16x16x4_f32 advances an output by four
+// FMAs in ascending lane group, so with lane group h feeding k = 8 h + q of a
+// 32-unit, MFMA q is the lane chain l[q] of 16 tokens x 16 weight rows (from
+// +0; a 64-long group goes on in the same accumulators).  A lane's weights of
+// a unit are one packed word, its activations two float4 of the a4 layout.
+// The lane sums and scale give a group's term, which goes to LDS; after the
+// barrier that ends a round of 8 gw groups (gw <= 4 a wave) a thread a (row,
+// token) adds the round's terms in group order, two term buffers, so the next
+// round's writes never meet these reads.  Loads run
+// two units ahead.  Bound by the f32 MFMAs (256 of about 460 clocks a unit)
+// and the VALU that forms the weights and the terms, on the same pipe; the
+// DPP-broadcast FMAs this replaced issue at half the plain rate.  16 rows with
+// the a4 copy, us before / now: 18432 x 2304 39.9 / 31.7, 2304 x 9216 31.7 /
+// 24.9, 4096 x 2304 14.5 / 10.0, 2304 x 2048 11.2 / 9.2, 512 x 512 6.1 / 6.1;
+// 3 rows cost the same.
+template <int G4>
+__global__ __launch_bounds__(512, 4) void i4_rows_mfma(const uint8_t* __restrict__ packed,
+                                                       const uint16_t* __restrict__ scale, int N, int K, int gw,
                                                        const float* __restrict__ a4, int M, float* __restrict__ out) {
     static_assert(G4 == 1 || G4 == 2, "a group is one or two 32-units");
-    constexpr int ND = 4 * NW;                 // DPP rows
-    constexpr int GPS = 3 - G4;                // groups a DPP row takes a slice (two steps a slice)
-    constexpr int SG = ND * GPS;               // groups a slice
-    constexpr int TS = SG + 1;                 // term row stride (floats), odd: conflict-free reads
-    constexpr int L = (16 * R + NW - 1) / NW;  // serial lanes a wave
-    static_assert(L <= 64, "one (row, token) pair a lane");
-    __shared__ float tb[2][16 * R][TS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int t = lane & 15, D = 4 * wave + (lane >> 4);
-    const int ng = K / (32 * G4), r0 = blockIdx.x * R;
-    const int nst = (ng + SG - 1) / SG * 2;  // unit steps: two a slice
-    const int sh = 4 * (t >> 2);
-    const size_t pitch = (size_t)K / 2;
-    const uint8_t* wrow[R];
-    const uint16_t* srow[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const size_t row = (size_t)min(r0 + r, N - 1);  // clamped: loads stay unconditional
-        wrow[r] = packed + row * pitch;
-        srow[r] = scale + row * ng;
-    }
-    const float* at = a4 + 4 * t;
-    // serial lane: pair p = wave L + lane -> (row p >> 4, token p & 15)
-    const int p = wave * L + lane;
-    const bool ser = lane < L && p < 16 * R;
-    float sum = 0.0f;
-    struct WB {
-        uint32_t w[R];
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    constexpr int P = 8;
+    __shared__ float tb[2][P * ROWS_GW][256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lh = lane >> 4;
+    const int ng = K / (32 * G4), R = P * gw, n0 = blockIdx.x * 16;
+    const size_t row = (size_t)min(n0 + li, N - 1);  // clamped: loads stay unconditional
+    const uint8_t* wp = packed + row * ((size_t)K / 2) + 4 * lh;
+    const uint16_t* sp = scale + row * ng;
+    const float* ap = a4 + 4 * li + 128 * lh;
+    // unit j of the wave: units j % G4 of its groups, gw adjacent ones a round
+    // (past the end the last group again)
+    const int rounds = (ng + R - 1) / R, nj = rounds * gw * G4;
+    int lg = wave * gw, lp = 0;  // the group to load next, its place in the round
+    auto unit = [&](int s) { return (size_t)(min(lg, ng - 1) * G4 + s); };
+    uint32_t w[2];
+    uint16_t sc[2];
+    f4v a[2][2];
+    auto load_w = [&](int u) {
+        w[u] = *reinterpret_cast<const uint32_t*>(wp + unit(G4 == 2 ? u : 0) * 16);
+        sc[u] = sp[min(lg, ng - 1)];
     };
-    struct AB {
-        float4 a[8];
-        uint32_t sc[R];
+    auto load_a = [&](int u) {  // and on
+        const float* q = ap + unit(G4 == 2 ? u : 0) * 512;
+        a[u][0] = *reinterpret_cast<const f4v*>(q);
+        a[u][1] = *reinterpret_cast<const f4v*>(q + 64);
+        if (G4 == 2 && u == 0) return;
+        const bool on = lp + 1 < gw;
+        lg += on ? 1 : 1 + R - gw;
+        lp = on ? lp + 1 : 0;
     };
-    // step j: slice j / 2; with G4 == 1 round j % 2 of the slice, with G4 == 2
-    // unit j % 2 of the DPP row's one group
-    auto group_of = [&](int j) { return (j >> 1) * SG + (G4 == 1 ? (j & 1) * ND : 0) + D; };
-    auto unit_of = [&](int j, int gi) { return min(gi, ng - 1) * G4 + (G4 == 2 ? (j & 1) : 0); };
-    auto load_w = [&](int j, WB& b) {
-        const uint32_t wo = (uint32_t)unit_of(j, group_of(j)) * 16 + 4 * (t & 3);
 #pragma unroll
-        for (int r = 0; r < R; ++r) b.w[r] = *reinterpret_cast<const uint32_t*>(wrow[r] + wo);
-    };
-    auto load_a = [&](int j, AB& b) {
-        const int gi = group_of(j);
-        const float* ap = at + (size_t)unit_of(j, gi) * 512;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) b.a[i] = *reinterpret_cast<const float4*>(ap + 64 * i);
-        const uint32_t so = 2 * (uint32_t)min(gi, ng - 1);
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            b.sc[r] = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(srow[r]) + so);
-    };
-    float l[R][8];  // each group's chains start with a product (dpp_fma16<., true>)
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) l[r][q] = 0.0f;  // defined inputs for the first asm
-    // ODD: the slice's second step, which ends every chain and the slice
-    auto step = [&](auto odd, int j, const WB& wb, const AB& ab) {
-        constexpr bool O = decltype(odd)::value;
-        constexpr bool START = G4 == 1 || !O;
-        float av[32];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            av[4 * i] = ab.a[i].x;
-            av[4 * i + 1] = ab.a[i].y;
-            av[4 * i + 2] = ab.a[i].z;
-            av[4 * i + 3] = ab.a[i].w;
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float w0 = (float)(int)__builtin_amdgcn_sbfe((int)wb.w[r], sh, 4);
-            const float w1 = (float)(int)__builtin_amdgcn_sbfe((int)wb.w[r], sh + 16, 4);
-            dpp_fma16<0, START>(l[r], w0, av);
-            dpp_fma16<1, START>(l[r], w1, av);
-        }
-        if constexpr (G4 == 2 && !O) return;  // the group goes on in the odd step
-        float(&tbs)[16 * R][TS] = tb[(j >> 1) & 1];
-        const int gi = group_of(j);
-        const int col = gi - (j >> 1) * SG;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float q0 = l[r][0] + l[r][4], q1 = l[r][1] + l[r][5], q2 = l[r][2] + l[r][6],
-                        q3 = l[r][3] + l[r][7];
-            const float term = h2f((uint16_t)ab.sc[r]) * ((q0 + q2) + (q1 + q3));
-            tbs[r * 16 + t][col] = gi < ng ? term : 0.0f;
-        }
-        if constexpr (!O) return;
-        __syncthreads();
-        if (ser) {
-            float v[SG];
-#pragma unroll
-            for (int i = 0; i < SG; ++i) v[i] = tbs[p][i];
-#pragma unroll
-            for (int i = 0; i < SG; ++i) sum = sum + v[i];
-        }
-    };
-    using T = std::true_type;
-    using F = std::false_type;
-    // The loads are unconditional (past the end: the last step again), so
-    // the wait for a step's data never covers a later one's, and fenced so
-    // that they issue before the step they run ahead of.
-    auto issued = [] {
-        asm volatile("" ::: "memory");
+    for (int u = 0; u < 2; ++u) {  // in the loop's order, so its waits count the same loads
+        load_w(u);
         __builtin_amdgcn_sched_barrier(0);
-    };
-    WB wc, wn, w2;
-    AB a0, a1;
-    load_w(0, wc);
-    load_a(0, a0);
-    load_w(1, wn);
-    for (int j = 0; j < nst; j += 2) {
-        load_w(min(j + 2, nst - 1), w2);
-        load_a(j + 1, a1);
-        issued();
-        step(F{}, j, wc, a0);
-        load_w(min(j + 3, nst - 1), wc);
-        load_a(min(j + 2, nst - 1), a0);
-        issued();
-        step(T{}, j + 1, wn, a1);
-        wn = wc;
-        wc = w2;
+        load_a(u);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    if (ser) {
-        const int pr = p >> 4, pt = p & 15;
-        if (pt < M && r0 + pr < N) out[(size_t)pt * N + r0 + pr] = sum;
+    float sum = 0.0f;  // tid < 256: token 4 (lane / 16) + tid / 64, row lane % 16
+    int r = 0, i = 0;
+    f4v l[8];
+    auto step = [&](auto uc) {
+        constexpr int u = decltype(uc)::value, s = G4 == 2 ? u : 0;
+        const int g = r * R + wave * gw + i;
+        float wv[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) wv[q] = (float)(int)__builtin_amdgcn_sbfe((int)w[u], 4 * q, 4);
+        const float sv = h2f(sc[u]);
+        load_w(u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const f4v c = s == 0 ? f4v{0.0f, 0.0f, 0.0f, 0.0f} : l[q];
+            l[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][q / 4][q % 4], wv[q], c, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_a(u);
+        if (s < G4 - 1) return;
+        float(&t)[P * ROWS_GW][256] = tb[r & 1];
+        if (g < ng) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float q0 = l[0][v] + l[4][v], q1 = l[1][v] + l[5][v], q2 = l[2][v] + l[6][v],
+                            q3 = l[3][v] + l[7][v];
+                t[wave * gw + i][64 * v + lane] = sv * ((q0 + q2) + (q1 + q3));
+            }
+        }
+        if (++i < gw) return;
+        __syncthreads();  // every wave ends the round here
+        if (wave < 4) {
+            const int n = min(R, ng - r * R);
+            int j = 0;
+            for (; j + 8 <= n; j += 8) {
+                float x[8];
+#pragma unroll
+                for (int v = 0; v < 8; ++v) x[v] = t[j + v][tid];
+#pragma unroll
+                for (int v = 0; v < 8; ++v) sum = sum + x[v];
+            }
+            for (; j < n; ++j) sum = sum + t[j][tid];
+        }
+        i = 0;
+        ++r;
+    };
+    for (int j = 0; j < nj; j += 2) {
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});  // past the last unit: no term (g >= ng), in every wave
+    }
+    if (wave < 4) {
+        const int tok = 4 * lh + wave, n = n0 + li;
+        if (tok < M && n < N) out[(size_t)tok * N + n] = sum;
     }
 }
 
@@ -1153,7 +1082,7 @@ hipError_t launch_i4_terms(const Weight& w, const float* a, float* out, hipStrea
 // Whether launch_i4_rows_a4 takes this weight (else launch_i4_m1_rows runs
 // the rows one M == 1 launch at a time).
 bool i4_rows_a4_ok(const Weight& w) {
-    return (w.g == 32 || w.g == 64) && w.k % w.g == 0 && w.k <= (size_t)INT32_MAX &&
+    return (w.g == 32 || w.g == 64) && w.k > 0 && w.k % w.g == 0 && w.k <= (size_t)INT32_MAX &&
            w.n <= (size_t)INT32_MAX && w.n * w.k / 2 < ((size_t)1 << 32);
 }
 
@@ -1165,31 +1094,20 @@ hipError_t launch_rows_to_a4(const float* a, size_t m, size_t k, float* a4, hipS
     return hipGetLastError();
 }
 
-namespace {
-template <int G4, int R>
-hipError_t rows_dpp(const Weight& w, int nw, size_t m, const float* a4, float* out, hipStream_t s) {
-    const unsigned grid = (unsigned)((w.n + R - 1) / R);
-    if (nw == 3)
-        i4_rows_dpp<G4, R, 3><<<dim3(grid), dim3(192), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, a4, (int)m, out);
-    else
-        i4_rows_dpp<G4, R, 4><<<dim3(grid), dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, a4, (int)m, out);
-    return hipGetLastError();
-}
-}  // namespace
-
 // m <= 16 rows in the a4 layout (launch_rows_to_a4), each in the M == 1
-// order.  Workgroups of 3 or 4 waves (12 or 16 DPP rows, whichever leaves
-// the fewer idle groups in the last slice; 4 on a tie) and 6 rows (each
-// activation register used 6 times) for wide outputs, 4 below 8192 rows,
-// where more workgroups matter more (measured on the Gemma-2 2B shapes).
+// order: the fewest rounds of 8 waves x ROWS_GW groups (64 KB of terms, two
+// workgroups a CU), the groups spread evenly over them (72: 3 rounds of 24).
 hipError_t launch_i4_rows_a4(const Weight& w, size_t m, const float* a4, float* out, hipStream_t s) {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (m > 16 || !i4_rows_a4_ok(w)) return hipErrorNotSupported;
-    const size_t ng = w.k / w.g, gps = w.g == 32 ? 2 : 1;  // groups a DPP row takes a slice
-    const int nw = (ng + 12 * gps - 1) / (12 * gps) * 12 < (ng + 16 * gps - 1) / (16 * gps) * 16 ? 3 : 4;
-    const bool r6 = w.n >= 8192;
-    if (w.g == 32) return r6 ? rows_dpp<1, 6>(w, nw, m, a4, out, s) : rows_dpp<1, 4>(w, nw, m, a4, out, s);
-    return r6 ? rows_dpp<2, 6>(w, nw, m, a4, out, s) : rows_dpp<2, 4>(w, nw, m, a4, out, s);
+    const size_t ng = w.k / w.g, rounds = (ng + 8 * ROWS_GW - 1) / (8 * ROWS_GW);
+    const int gw = rounds ? (int)((ng + 8 * rounds - 1) / (8 * rounds)) : 1;
+    const unsigned grid = (unsigned)((w.n + 15) / 16);
+    if (w.g == 32)
+        i4_rows_mfma<1><<<dim3(grid), dim3(512), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, gw, a4, (int)m, out);
+    else
+        i4_rows_mfma<2><<<dim3(grid), dim3(512), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, gw, a4, (int)m, out);
+    return hipGetLastError();
 }
 
 // m rows, each in the M == 1 order (bit-identical to m launches at M == 1);
