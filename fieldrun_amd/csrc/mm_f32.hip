@@ -131,15 +131,15 @@ struct Packed {
             const int r = TT * t + lane % TT;
             const v4u q = w4[r * 4 + (c ^ ((r >> 2) & 3))];
             const uint32_t w[4] = {q.x >> (4 * h), q.y >> (4 * h), q.z >> (4 * h), q.w >> (4 * h)};
-            const float sc = sl[c * R + r], mi = Q ? sl[(4 + c) * R + r] : -1032.0f * sc;
+            const float sc = sl[c * R + r], mi = Q ? sl[(4 + c) * R + r] : 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {  // word i: k = 8 i + h and 8 i + 4 + h, nibble h of each half
                 if constexpr (Q) {  // u as f16 pairs, then scale * u (exact) + min in one rounding
                     const h2v u = __builtin_bit_cast(h2v, (w[i] & 0x000F000Fu) | 0x64006400u) - h2v{1024, 1024};
                     x[t][2 * i] = __builtin_fmaf((float)u.x, sc, mi);
                     x[t][2 * i + 1] = __builtin_fmaf((float)u.y, sc, mi);
-                } else {  // the f16 1032 + s4, then (1032 + s4) * scale - 1032 * scale: exact
-                    const h2v u = __builtin_bit_cast(h2v, (w[i] & 0x000F000Fu) ^ 0x64086408u);
+                } else {  // s4 from the f16 1032 + s4, then one product: exact, and s4 * scale for any scale
+                    const h2v u = __builtin_bit_cast(h2v, (w[i] & 0x000F000Fu) ^ 0x64086408u) - h2v{1032, 1032};
                     x[t][2 * i] = __builtin_fmaf((float)u.x, sc, mi);
                     x[t][2 * i + 1] = __builtin_fmaf((float)u.y, sc, mi);
                 }

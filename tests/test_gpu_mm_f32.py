@@ -54,6 +54,31 @@ def test_non_finite_and_subnormal_values(ctx):
     same(got[fin], ref[fin])
 
 
+@pytest.mark.parametrize("g,k", [(32, 40), (64, 200), (48, 104), (32, 320)])
+@pytest.mark.parametrize("m,n", [(2, 16), (33, 70)])
+def test_non_finite_scales(ctx, m, n, k, g):
+    """A group scale that is infinite or NaN: s4 * scale in each weight, so a
+    group whose products share a sign sums to that infinity (the short last
+    group of rows of one nibble, whose activations are positive), a zero
+    nibble or both signs to NaN."""
+    rng = np.random.default_rng(m + n + k + g)
+    a = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
+    q, s, mn = packed_weight(rng, n, k, g)
+    last = (k - 1) // g
+    for row, (scale, byte) in enumerate([(np.inf, 0x33), (np.inf, 0xDD), (-np.inf, 0x33), (-np.inf, 0x88), (np.inf, 0x30),
+                                         (np.nan, 0x33), (np.inf, 0x3D), (-np.inf, 0x7F)]):
+        q[row, last * g // 2:] = byte
+        s[row, last] = scale
+    s[8, 0], s[9, 0] = np.inf, np.nan  # a whole group of mixed nibbles
+    f32 = lambda v: v.astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        for got, ref in ((ctx.upload_i4(q, s, k, g).mm_exact(a), oracle.mm_i4(a, q, f32(s), k, g)),
+                         (ctx.upload_q4a(q, s, mn, k, g).mm(a), oracle.mm_q4a(a, q, f32(s), f32(mn), k, g))):
+            assert np.isinf(ref[:, :4]).all() and np.isnan(ref[:, 5]).all()
+            assert np.array_equal(np.isnan(got), np.isnan(ref))
+            same(got[~np.isnan(ref)], ref[~np.isnan(ref)])
+
+
 @pytest.mark.parametrize("dtype", ["f16", "f32", "q4a", "i4"])
 @pytest.mark.parametrize("T,topk,d,mi", [(1, 2, 288, 70), (4, 2, 96, 33), (5, 3, 256, 17), (90, 2, 520, 64),
                                          (200, 1, 64, 300)])
