@@ -253,8 +253,9 @@ hipError_t launch_m(const Weight& w, size_t m, const int8_t* a8, const float* sa
 // estimate of 30 us the tiles are faster (K=896 N=4864 M=129: 18 against 61;
 // K=4864 N=896: 18 against 42; K=4096 N=14336 M=48: 28 against 34, M=129
 // estimated at 90: 71 against 41).
+// The GEMM's limit stays: K to 20480.
 bool mid_i8_ok(const Weight& w, size_t m) {
-    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64) return false;
+    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64 || w.kp > 20480) return false;
     const double tiles = (double)((w.n + 15) / 16) * (double)((m + 15) / 16);
     return tiles * (3.2 + 0.0019 * (double)w.kp) <= 30000.0;
 }

@@ -92,6 +92,19 @@ def test_i8_gemm_acc_exact_out_within_tol(ctx, m, k, n):
     assert rel.max() <= 1e-5
 
 
+def test_i8_long_rows_of_prompts_are_refused(ctx):
+    """More than 16 rows of K beyond 20480 are refused at any N (the decode
+    kernels take such rows), and the context stays usable."""
+    import fieldrun_amd as fa
+    for m, k, n in ((17, 20481, 64), (40, 24576, 300)):
+        a, wt, scale = case(m, k, n, 900 + m)
+        w = ctx.upload_i8(wt, scale)
+        with pytest.raises(fa.FrqError):
+            w.mm(a)
+        got = w.mm(a[:3])
+        assert np.array_equal(got.view(np.uint32), oracle.mm_i8(a[:3], wt, scale).view(np.uint32))
+
+
 def test_i8_activation_edge_cases(ctx):
     k, n = 200, 96
     wt, scale = synth.int8_weight(n, k, 7)
