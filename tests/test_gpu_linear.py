@@ -33,6 +33,19 @@ def check_quant(a, a8, sa, oi, ov):
         assert np.array_equal(ov[i, :t].view(np.uint32), qov.view(np.uint32)), f"oval row {i}"
 
 
+# Products above the cut of the one-pass int8 tiles (skinny_i8.hip), so on the
+# MFMA GEMM: ragged M, N and K, the exact epilogue's 16-, 8- and 4-column
+# forms by K, K below the outlier count.
+GEMM_SHAPES = [(515, 1000, 6001), (300, 5000, 4001), (130, 18944, 3001), (2000, 20, 5000), (700, 37, 9001)]
+
+
+def takes_gemm(out, ref):
+    """Whether frq_mm's outputs come from the GEMM: its union correction
+    rounds some outputs otherwise than the reference's order, which the
+    kernels for fewer rows keep bit for bit."""
+    return not np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+
+
 def corr_mag(a, wt, scale, acc):
     mags = []
     for i in range(a.shape[0]):
@@ -61,24 +74,30 @@ def test_i8_gemv_bit_exact(ctx, m, k, n):
 
 @pytest.mark.parametrize("m,k,n", [(17, 896, 4864), (130, 512, 301), (64, 37, 50), (20, 20, 30), (200, 128, 129),
                                    (1024, 3584, 512), (300, 5000, 257), (600, 18944, 300), (40, 20480, 64),
-                                   (2048, 4096, 256), (1100, 1000, 1001)])
+                                   (2048, 4096, 256), (1100, 1000, 1001), *GEMM_SHAPES])
 def test_i8_mm_exact_bit_exact(ctx, m, k, n):
-    """frq_mm_exact_dev at M > 16: the GEMM's exact int32 sums, then the
-    M > 1 arm's sequential outlier correction with every column block's
-    weights in LDS (16, 8 or 4 columns by K; ragged N and M, K below the
-    outlier count), bit for bit against the oracle."""
+    """frq_mm_exact_dev at M > 16, bit for bit against the oracle.  The
+    products of GEMM_SHAPES take the GEMM's exact int32 sums, then the M > 1
+    arm's sequential outlier correction with every column block's weights in
+    LDS (16, 8 or 4 columns by K; ragged N and M, K below the outlier count);
+    the smaller ones the one-pass tiles."""
     a, wt, scale = case(m, k, n, 300 + m + k + n)
     w = ctx.upload_i8(wt, scale)
     ref = oracle.mm_i8_mt(a, wt, scale, 16)
     got = w.mm_exact(a)
     bad = np.argwhere(got.view(np.uint32) != ref.view(np.uint32))
     assert len(bad) == 0, (len(bad), bad[:4].tolist())
+    if (m, k, n) in GEMM_SHAPES:
+        assert takes_gemm(w.mm(a), ref)
 
 
 @pytest.mark.parametrize("m,k,n", [(5, 896, 4864), (16, 4096, 1024), (128, 896, 640), (130, 512, 300),
                                    (64, 37, 50), (16, 14336, 256), (33, 4864, 896), (200, 128, 129),
-                                   (128, 14336, 512), (2048, 128, 14336)])
+                                   (128, 14336, 512), (2048, 128, 14336), *GEMM_SHAPES])
 def test_i8_gemm_acc_exact_out_within_tol(ctx, m, k, n):
+    """Sums bit-exact and outputs within the bar at M > 1: the skinny and
+    one-pass kernels at the smaller products, the GEMM with the union
+    correction at GEMM_SHAPES and 2048 x 128 x 14336."""
     a, wt, scale = case(m, k, n, 200 + m + k + n)
     w = ctx.upload_i8(wt, scale)
     out, acc, a8, sa, oi, ov = w.mm_debug(a)
@@ -90,6 +109,8 @@ def test_i8_gemm_acc_exact_out_within_tol(ctx, m, k, n):
     assert np.all(err <= 1e-6 * mag + 1e-30), float((err / (mag + 1e-30)).max())
     rel = err.max(axis=1) / np.abs(ref).max(axis=1)
     assert rel.max() <= 1e-5
+    if (m, k, n) in GEMM_SHAPES:
+        assert takes_gemm(out, ref)
 
 
 def test_i8_long_rows_of_prompts_are_refused(ctx):
@@ -264,9 +285,10 @@ def test_i4_reference_kat_through_gpu(ctx):
     assert w.mm(np.ones((1, 4), np.float32))[0, 0] == 1.0
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 896, 4864), (3, 4096, 300), (40, 896, 640), (300, 4864, 896)])
+@pytest.mark.parametrize("m,k,n", [(1, 896, 4864), (3, 4096, 300), (40, 896, 640), (300, 4864, 896),
+                                   (515, 1000, 6001), (130, 18944, 3001)])
 def test_i8_device_entry_points_match_host(ctx, m, k, n):
-    """frq_quant_i8_dev + frq_mm_i8_q_dev (device pointers, row-major a8 of
+    """(The last two on the GEMM.)  frq_quant_i8_dev + frq_mm_i8_q_dev (device pointers, row-major a8 of
     pitch frq_quant_pitch(K)) give the same bits as frq_mm_i8_debug."""
     import fieldrun_amd as fa
     from fieldrun_amd import hip
