@@ -246,18 +246,26 @@ hipError_t launch_m(const Weight& w, size_t m, const int8_t* a8, const float* sa
 
 }  // namespace
 
-// A 16 x 16 tile costs about 3.2 ns + 1.9 ps a k over the whole card
-// (measured for K 512 .. 14336, N 512 .. 30000, M 20 .. 512), the MFMA GEMM
-// with its correction 33 us at the least (the pre-pass, the split sums and the
-// epilogue), 60 .. 78 where K <= 2048 makes the outlier union dense: up to an
-// estimate of 30 us the tiles are faster (K=896 N=4864 M=129: 18 against 61;
-// K=4864 N=896: 18 against 42; K=4096 N=14336 M=48: 28 against 34, M=129
-// estimated at 90: 71 against 41).
-// The GEMM's limit stays: K to 20480.
+// The middling batches that this kernel takes from the GEMM (with the union
+// correction for frq_mm_dev, with the exact epilogue for frq_mm_exact_dev):
+// by an estimate of its tiles, 3.2 ns + 1.9 ps a k each over the whole card,
+// up to 30 us.  Its time is that and 6 .. 12 us (the quant and the launches;
+// at long K the walk of one wave, which the estimate leaves out: 64 us at 32 x
+// 18944 x 3584, estimated at 18), the GEMM's at least 34 us from K = 512 on and
+// more with K (56 at 9216, 75 at 18944; 77 at that product), so the tiles are
+// the faster there; a higher cut would still gain (512 x 896 x 4864: 48
+// against 68).  Shorter K is cheap for the GEMM (K = 128:
+// 24 us however many rows, 256: 28), and outputs wider than 32768 run half-empty
+// workgroups in a third round (32 x 512 x 40000: 43 against 34 exact).  Timed on
+// both routes at 1800 products of K 32 .. 20480, N 64 .. 65000, M 17 .. 4096:
+// none that this rule picks is slower by more than 7% (K = 384; 3% from 512).
+// The GEMM's limits stay: K to 20480.
 bool mid_i8_ok(const Weight& w, size_t m) {
-    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64 || w.kp > 20480) return false;
+    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64 || w.kp > 20480 || w.n > 32768)
+        return false;
     const double tiles = (double)((w.n + 15) / 16) * (double)((m + 15) / 16);
-    return tiles * (3.2 + 0.0019 * (double)w.kp) <= 30000.0;
+    const double cut = w.kp < 256 ? 13000.0 : w.kp < 512 ? 17000.0 : 30000.0;
+    return tiles * (3.2 + 0.0019 * (double)w.kp) <= cut;
 }
 
 hipError_t launch_mid_i8(const Weight& w, size_t m, const int8_t* a8, const float* sa, const uint32_t* oidx,

@@ -35,8 +35,9 @@ def check_quant(a, a8, sa, oi, ov):
 
 # Products above the cut of the one-pass int8 tiles (skinny_i8.hip), so on the
 # MFMA GEMM: ragged M, N and K, the exact epilogue's 16-, 8- and 4-column
-# forms by K, K below the outlier count.
-GEMM_SHAPES = [(515, 1000, 6001), (300, 5000, 4001), (130, 18944, 3001), (2000, 20, 5000), (700, 37, 9001)]
+# forms by K, K below the outlier count, outputs too wide for the tiles.
+GEMM_SHAPES = [(515, 1000, 6001), (300, 5000, 4001), (130, 18944, 3001), (2000, 20, 5000), (700, 37, 9001),
+               (20, 600, 33001), (400, 128, 5001)]
 
 
 def takes_gemm(out, ref):
