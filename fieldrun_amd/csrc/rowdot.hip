@@ -233,12 +233,20 @@ __global__ __launch_bounds__(64 * WPB) void rowdot_kernel(
 template <int DT, bool ARG>
 hipError_t launch_dt(const Weight& w, const float* x, const int64_t* cand, size_t nout, float* out,
                      unsigned long long* best, int* err, hipStream_t s) {
-    // At most one wave a SIMD: workgroups of one wave, over all the CUs, and
-    // six chunks in flight (16384 x 3584 f16: 64 -> 48 us; four-wave
+    // At most half a wave a SIMD: workgroups of one wave, over all the CUs,
+    // and six chunks in flight (16384 x 3584 f16: 64 -> 48 us; four-wave
     // workgroups leave three CUs in four idle there).  Up to about four waves
-    // per SIMD: three chunks (latency-bound), else two (the occupancy carries
-    // the load).
-    const bool few = nout <= 1024 * 64, deep = nout < 4 * 1024 * 64;
+    // per SIMD: four-wave workgroups and three chunks (latency-bound), else
+    // two (the occupancy carries the load).  Where the one-wave form ends, us
+    // one-wave / three chunks: 32768 x 896 f16 17.5 / 19.4, 40000 x 896 19.8 /
+    // 19.4, 50257 x 768 19.1 / 16.9, 65536 x 896 24.8 / 20.6; rows of 2048 and
+    // more a little later (40000 x 2304 38.3 / 41.9, 50257 x 2304 44.0 / 41.9).
+    // Whole-table rows a multiple of 8 KB apart meet the same memory channels
+    // at each step, which more rows in flight make worse: 4000 x 4096 f16 53 /
+    // 73, but 8000 84 / 73 and 28000 108 / 74; f32 8000 x 4096 52 / 79, 28000
+    // x 4096 111 / 104.
+    const bool aligned = !cand && w.rpitch % 8192 == 0 && nout > (DT == 0 ? 8192 : 4096);
+    const bool few = nout <= (w.k >= 2048 ? 640 : 512) * (size_t)64 && !aligned, deep = nout < 4 * 1024 * 64;
 #define FRQ_ROWDOT(SUBV, DEPTHV, WPBV)                                                                   \
     rowdot_kernel<DT, SUBV, DEPTHV, WPBV, ARG>                                                           \
         <<<dim3((unsigned)((nout + 64 * WPBV - 1) / (64 * WPBV))), dim3(64 * WPBV), 0, s>>>(             \

@@ -55,6 +55,22 @@ def test_rowdot_bit_exact(ctx, kind, rows, d):
     t.free()
 
 
+@pytest.mark.parametrize("kind,rows,d", [("f16", 32768, 40), ("f16", 32769, 40), ("rowi8", 40960, 2050),
+                                         ("rowi8", 40961, 2050), ("f16", 4096, 4096), ("f16", 4097, 4096),
+                                         ("f32", 8193, 2048), ("rowi8", 4100, 8192)])
+def test_rowdot_at_the_borders_of_its_forms(ctx, kind, rows, d):
+    """Either side of where one-wave workgroups give way to four-wave ones:
+    by rows, for rows of 2048 elements and more, and for rows a multiple of
+    8 KB apart (the subset keeps the one-wave form there)."""
+    data, scale = table(kind, rows, d, rows + d)
+    x = np.random.default_rng(d).standard_normal(d).astype(np.float32)
+    t = ctx.upload_rows(kind, data, scale)
+    assert same_bits(t.rowdot_f32(x), oracle.rowdot_f32(kind, oracle_data(kind, data), x, scale))
+    cand = np.random.default_rng(rows).integers(0, rows, 4200)
+    assert same_bits(t.rowdot_f32_subset(x, cand), oracle.rowdot_f32_subset(kind, oracle_data(kind, data), x, cand, scale))
+    t.free()
+
+
 def test_rowdot_gpt2_vocab_device_entry_points(ctx):
     rows, d = 50257, 768
     data, _ = table("f16", rows, d, 5)
