@@ -33,7 +33,8 @@
 // and invalidate the whole L2.
 // Other shapes run i4_gemv_generic (M == 1, bit-identical to i4_dot_avx2)
 // or, M > 1 in the exact order, the f32 matrix cores (mm_f32.hip).  Up to 16
-// independent M == 1 rows (a batched decode) run i4_rows_mfma.
+// independent M == 1 rows (a batched decode) run i4_rows_mfma, of narrow
+// outputs i4_rows_dpp.
 #include "frq_internal.h"
 
 namespace frq {
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(NT) void i4_m1_stream(const uint8_t* __restrict__ p
 
 constexpr int ROWS_GW = 4;  // groups a wave of i4_rows_mfma takes a round, at most
 
-// The activation layout of i4_rows_mfma: the 16 token rows interleaved by
+// The activation layout of i4_rows_mfma and i4_rows_dpp: the 16 token rows interleaved by
 // k-quads, a4[64 (k / 4) + 4 t + k % 4] = a[t][k] (rows t >= M zero), so
 // that 16 token lanes read 256 contiguous bytes a load.
 __global__ void rows_to_a4_kernel(const float* __restrict__ a, int M, int K, float* __restrict__ a4) {
@@ -342,6 +343,199 @@ __global__ void rows_to_a4_kernel(const float* __restrict__ a, int M, int K, flo
     float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (t < M) v = *reinterpret_cast<const float4*>(a + (size_t)t * K + 4 * kq);
     reinterpret_cast<float4*>(a4)[i] = v;
+}
+
+// 16 FMAs of one weight register v of a 32-unit into lane chains
+// l[4 v .. 4 v + 3]: v_fmac_f32_dpp with row_newbcast:n gives each token
+// lane of a 16-lane DPP row the weight held by lane n of that row.  Lane n
+// holds element e = 8 (n & 3) + (n >> 2) + 4 v, which is nibble
+// (n >> 2) + 4 v of word n & 3 (chain q = e & 7, chunk c = e >> 3), and its
+// product takes av[e]; the FMAs go c-major so each chain advances in chunk
+// order.  START begins the chains: chunk 0 is a v_mul_f32_dpp, which
+// differs from fma(w, a, +0) only in giving -0 for a -0 product; a chain
+// is exact otherwise, the lane sums of i4_dot_avx2 then differ at most in
+// the sign of a zero, and so does a group term, which the running sum from
+// +0 absorbs (+0 + -0 == +0): the row sums are bit-identical.  The s_nop
+// gives the two wait states a DPP read needs after the VALU write of w,
+// which the compiler does not see inside the asm.
+#define FRQ_DPPF(op, acc, n, src) #op "_f32_dpp %" #acc ", %4, %" #src " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
+#define FRQ_DPP_C0(op) FRQ_DPPF(op, 0, 0, 5) FRQ_DPPF(op, 1, 4, 9) FRQ_DPPF(op, 2, 8, 13) FRQ_DPPF(op, 3, 12, 17)
+#define FRQ_DPP_C123                                                                                          \
+    FRQ_DPPF(v_fmac, 0, 1, 6) FRQ_DPPF(v_fmac, 1, 5, 10) FRQ_DPPF(v_fmac, 2, 9, 14) FRQ_DPPF(v_fmac, 3, 13, 18) \
+    FRQ_DPPF(v_fmac, 0, 2, 7) FRQ_DPPF(v_fmac, 1, 6, 11) FRQ_DPPF(v_fmac, 2, 10, 15)                            \
+    FRQ_DPPF(v_fmac, 3, 14, 19) FRQ_DPPF(v_fmac, 0, 3, 8) FRQ_DPPF(v_fmac, 1, 7, 12)                            \
+    FRQ_DPPF(v_fmac, 2, 11, 16) FRQ_DPPF(v_fmac, 3, 15, 20)
+#define FRQ_DPP_OPS(V)                                                                              \
+    : "+v"(l[4 * V]), "+v"(l[4 * V + 1]), "+v"(l[4 * V + 2]), "+v"(l[4 * V + 3])                    \
+    : "v"(w), "v"(av[4 * V]), "v"(av[8 + 4 * V]), "v"(av[16 + 4 * V]), "v"(av[24 + 4 * V]),         \
+      "v"(av[1 + 4 * V]), "v"(av[9 + 4 * V]), "v"(av[17 + 4 * V]), "v"(av[25 + 4 * V]),             \
+      "v"(av[2 + 4 * V]), "v"(av[10 + 4 * V]), "v"(av[18 + 4 * V]), "v"(av[26 + 4 * V]),            \
+      "v"(av[3 + 4 * V]), "v"(av[11 + 4 * V]), "v"(av[19 + 4 * V]), "v"(av[27 + 4 * V])
+template <int V, bool START>
+__device__ __forceinline__ void dpp_fma16(float (&l)[8], float w, const float (&av)[32]) {
+    if constexpr (START)
+        asm("s_nop 1\n\t" FRQ_DPP_C0(v_mul) FRQ_DPP_C123 FRQ_DPP_OPS(V));
+    else
+        asm("s_nop 1\n\t" FRQ_DPP_C0(v_fmac) FRQ_DPP_C123 FRQ_DPP_OPS(V));
+}
+#undef FRQ_DPP_OPS
+#undef FRQ_DPP_C123
+#undef FRQ_DPP_C0
+#undef FRQ_DPPF
+
+// M independent rows (M <= 16), each in the M == 1 order (i4_dot_avx2),
+// with the weights broadcast across tokens: lane 16 d + t of a wave is token
+// t in DPP row d, and the workgroup's ND = 4 NW DPP rows D = 4 wave + d take
+// a slice of 2 ND groups in two rounds (groups 2 ND s + ND i + D, i = 0, 1).
+// A lane holds its token's 32 activations of the current 32-unit (read from
+// the a4 layout) and, for each of the workgroup's R weight rows, the packed
+// word t & 3 of the unit, whose nibbles t >> 2 and 4 + (t >> 2) become its
+// two f32 weight registers (dpp_fma16): each activation register serves R
+// rows and each weight register 16 tokens.  A group's term scale * gsum goes
+// to LDS (+0 for the groups past the end, which the running sum absorbs
+// exactly: it is never -0); after the slice's one barrier the lane of (row,
+// token) adds the slice's 2 ND terms to its running sum in group order (two
+// term buffers, so the next slice's writes never meet this slice's reads).
+// Activations and scales are loaded one step ahead, weights two.  Needs
+// K % (32 G4) == 0.  Bound by the DPP FMAs' issue.  It takes the narrow
+// outputs, where the 16-row tiles of i4_rows_mfma leave most CUs idle and
+// these 4-row ones do not; 16 rows, us here / there: 896 x 4864 12.3 / 14.8,
+// 512 x 9216 (groups of 64) 15.6 / 22.6, 512 x 2304 8.5 / 9.9; from a second
+// workgroup a CU on it loses (1536 x 2304 10.6 / 10.0, 2304 x 4864 20.3 /
+// 14.8).
+template <int G4, int NW>
+__global__ __launch_bounds__(64 * NW) void i4_rows_dpp(const uint8_t* __restrict__ packed,
+                                                       const uint16_t* __restrict__ scale, int N, int K,
+                                                       const float* __restrict__ a4, int M, float* __restrict__ out) {
+    static_assert(G4 == 1 || G4 == 2, "a group is one or two 32-units");
+    constexpr int R = 4;                       // weight rows a workgroup
+    constexpr int ND = 4 * NW;                 // DPP rows
+    constexpr int GPS = 3 - G4;                // groups a DPP row takes a slice (two steps a slice)
+    constexpr int SG = ND * GPS;               // groups a slice
+    constexpr int TS = SG + 1;                 // term row stride (floats), odd: conflict-free reads
+    constexpr int L = (16 * R + NW - 1) / NW;  // serial lanes a wave
+    static_assert(L <= 64, "one (row, token) pair a lane");
+    __shared__ float tb[2][16 * R][TS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int t = lane & 15, D = 4 * wave + (lane >> 4);
+    const int ng = K / (32 * G4), r0 = blockIdx.x * R;
+    const int nst = (ng + SG - 1) / SG * 2;  // unit steps: two a slice
+    const int sh = 4 * (t >> 2);
+    const size_t pitch = (size_t)K / 2;
+    const uint8_t* wrow[R];
+    const uint16_t* srow[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const size_t row = (size_t)min(r0 + r, N - 1);  // clamped: loads stay unconditional
+        wrow[r] = packed + row * pitch;
+        srow[r] = scale + row * ng;
+    }
+    const float* at = a4 + 4 * t;
+    // serial lane: pair p = wave L + lane -> (row p >> 4, token p & 15)
+    const int p = wave * L + lane;
+    const bool ser = lane < L && p < 16 * R;
+    float sum = 0.0f;
+    struct WB {
+        uint32_t w[R];
+    };
+    struct AB {
+        float4 a[8];
+        uint32_t sc[R];
+    };
+    // step j: slice j / 2; with G4 == 1 round j % 2 of the slice, with G4 == 2
+    // unit j % 2 of the DPP row's one group
+    auto group_of = [&](int j) { return (j >> 1) * SG + (G4 == 1 ? (j & 1) * ND : 0) + D; };
+    auto unit_of = [&](int j, int gi) { return min(gi, ng - 1) * G4 + (G4 == 2 ? (j & 1) : 0); };
+    auto load_w = [&](int j, WB& b) {
+        const uint32_t wo = (uint32_t)unit_of(j, group_of(j)) * 16 + 4 * (t & 3);
+#pragma unroll
+        for (int r = 0; r < R; ++r) b.w[r] = *reinterpret_cast<const uint32_t*>(wrow[r] + wo);
+    };
+    auto load_a = [&](int j, AB& b) {
+        const int gi = group_of(j);
+        const float* ap = at + (size_t)unit_of(j, gi) * 512;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) b.a[i] = *reinterpret_cast<const float4*>(ap + 64 * i);
+        const uint32_t so = 2 * (uint32_t)min(gi, ng - 1);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            b.sc[r] = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(srow[r]) + so);
+    };
+    float l[R][8];  // each group's chains start with a product (dpp_fma16<., true>)
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) l[r][q] = 0.0f;  // defined inputs for the first asm
+    // ODD: the slice's second step, which ends every chain and the slice
+    auto step = [&](auto odd, int j, const WB& wb, const AB& ab) {
+        constexpr bool O = decltype(odd)::value;
+        constexpr bool START = G4 == 1 || !O;
+        float av[32];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            av[4 * i] = ab.a[i].x;
+            av[4 * i + 1] = ab.a[i].y;
+            av[4 * i + 2] = ab.a[i].z;
+            av[4 * i + 3] = ab.a[i].w;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float w0 = (float)(int)__builtin_amdgcn_sbfe((int)wb.w[r], sh, 4);
+            const float w1 = (float)(int)__builtin_amdgcn_sbfe((int)wb.w[r], sh + 16, 4);
+            dpp_fma16<0, START>(l[r], w0, av);
+            dpp_fma16<1, START>(l[r], w1, av);
+        }
+        if constexpr (G4 == 2 && !O) return;  // the group goes on in the odd step
+        float(&tbs)[16 * R][TS] = tb[(j >> 1) & 1];
+        const int gi = group_of(j);
+        const int col = gi - (j >> 1) * SG;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float q0 = l[r][0] + l[r][4], q1 = l[r][1] + l[r][5], q2 = l[r][2] + l[r][6],
+                        q3 = l[r][3] + l[r][7];
+            const float term = h2f((uint16_t)ab.sc[r]) * ((q0 + q2) + (q1 + q3));
+            tbs[r * 16 + t][col] = gi < ng ? term : 0.0f;
+        }
+        if constexpr (!O) return;
+        __syncthreads();
+        if (ser) {
+            float v[SG];
+#pragma unroll
+            for (int i = 0; i < SG; ++i) v[i] = tbs[p][i];
+#pragma unroll
+            for (int i = 0; i < SG; ++i) sum = sum + v[i];
+        }
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    // The loads are unconditional (past the end: the last step again), so
+    // the wait for a step's data never covers a later one's, and fenced so
+    // that they issue before the step they run ahead of.
+    auto issued = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    WB wc, wn, w2;
+    AB a0, a1;
+    load_w(0, wc);
+    load_a(0, a0);
+    load_w(1, wn);
+    for (int j = 0; j < nst; j += 2) {
+        load_w(min(j + 2, nst - 1), w2);
+        load_a(j + 1, a1);
+        issued();
+        step(F{}, j, wc, a0);
+        load_w(min(j + 3, nst - 1), wc);
+        load_a(min(j + 2, nst - 1), a0);
+        issued();
+        step(T{}, j + 1, wn, a1);
+        wn = wc;
+        wc = w2;
+    }
+    if (ser) {
+        const int pr = p >> 4, pt = p & 15;
+        if (pt < M && r0 + pr < N) out[(size_t)pt * N + r0 + pr] = sum;
+    }
 }
 
 // M independent rows (M <= 16), each in the M == 1 order (i4_dot_avx2), on
@@ -1094,12 +1288,30 @@ hipError_t launch_rows_to_a4(const float* a, size_t m, size_t k, float* a4, hipS
     return hipGetLastError();
 }
 
+namespace {
+// Workgroups of 3 or 4 waves (12 or 16 DPP rows), whichever leaves the fewer
+// idle groups in the last slice; 4 on a tie.
+template <int G4>
+hipError_t rows_dpp(const Weight& w, size_t m, const float* a4, float* out, hipStream_t s) {
+    const size_t ng = w.k / w.g, gps = 3 - G4;  // groups a DPP row takes a slice
+    const unsigned grid = (unsigned)((w.n + 3) / 4);
+    if ((ng + 12 * gps - 1) / (12 * gps) * 12 < (ng + 16 * gps - 1) / (16 * gps) * 16)
+        i4_rows_dpp<G4, 3><<<dim3(grid), dim3(192), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, a4, (int)m, out);
+    else
+        i4_rows_dpp<G4, 4><<<dim3(grid), dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k, a4, (int)m, out);
+    return hipGetLastError();
+}
+}  // namespace
+
 // m <= 16 rows in the a4 layout (launch_rows_to_a4), each in the M == 1
-// order: the fewest rounds of 8 waves x ROWS_GW groups (64 KB of terms, two
-// workgroups a CU), the groups spread evenly over them (72: 3 rounds of 24).
+// order.  Narrow outputs take i4_rows_dpp; i4_rows_mfma the fewest rounds of 8 waves x ROWS_GW groups
+// (64 KB of terms, two workgroups a CU), the groups spread evenly over them
+// (72: 3 rounds of 24).
 hipError_t launch_i4_rows_a4(const Weight& w, size_t m, const float* a4, float* out, hipStream_t s) {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (m > 16 || !i4_rows_a4_ok(w)) return hipErrorNotSupported;
+    if (w.n <= 4 * (size_t)device_cus(w.device))  // i4_rows_dpp's workgroups in one round
+        return w.g == 32 ? rows_dpp<1>(w, m, a4, out, s) : rows_dpp<2>(w, m, a4, out, s);
     const size_t ng = w.k / w.g, rounds = (ng + 8 * ROWS_GW - 1) / (8 * ROWS_GW);
     const int gw = rounds ? (int)((ng + 8 * rounds - 1) / (8 * rounds)) : 1;
     const unsigned grid = (unsigned)((w.n + 15) / 16);

@@ -45,6 +45,9 @@ SHAPES = [
     # 16), row counts off the workgroup's, both group sizes
     (1, 300, 2048, 32), (3, 257, 96, 32), (5, 1000, 4160, 64), (8, 33, 64, 64),
     (12, 700, 1536, 64), (15, 2311, 800, 32), (16, 4, 32, 32), (2, 5000, 512, 64),
+    # ... around 1024 rows, where the 4-row tiles give way to the 16-row ones
+    (16, 896, 4864, 32), (16, 1024, 2336, 32), (7, 1025, 2336, 32), (16, 1030, 4160, 64), (3, 1100, 32, 32),
+    (5, 1200, 64, 64), (16, 1023, 3072, 64),
 ]
 
 
@@ -85,6 +88,20 @@ def test_i4_rows_nonfinite(ctx):
     w = ctx.upload_i4(packed, s16, k, g)
     out, ref = w.mm_rows(a), per_row(w, a)
     assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+    w.free()
+
+
+def test_i4_rows_nonfinite_wide(ctx):
+    """The same on the 16-row tiles (more than 1024 rows)."""
+    m, n, k, g = 6, 1100, 1024, 32
+    packed, s16 = raw_i4(n, k, g, 7402)
+    a = acts(m, k, 7403)
+    a[0, 5], a[4, 700], a[5, 3] = np.inf, -np.inf, np.nan
+    w = ctx.upload_i4(packed, s16, k, g)
+    out, ref = w.mm_rows(a), per_row(w, a)
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    fin = ~np.isnan(ref)
+    assert np.array_equal(out[fin].view(np.uint32), ref[fin].view(np.uint32))
     w.free()
 
 
