@@ -99,8 +99,9 @@ __global__ void i4_gemv_generic(const uint8_t* __restrict__ packed,
 // the activation row in LDS (36 floats a 32, so lanes a group apart meet
 // other banks), and a lane a row adding its group terms in order.  Bound by
 // the VALU at wide outputs and by the latency of a group's chain at narrow
-// ones; a thread a row instead (i4_gemv_generic, kept where LDS does not hold
-// the row and its terms) walks all of K alone: 184 x 6346 334 -> 8 us.
+// ones; a thread a row instead (i4_gemv_generic, kept up to K = 64 and where
+// LDS does not hold the row and its terms) walks all of K alone: 184 x 6346
+// 334 -> 8 us.  q4a keeps its own form at most sizes (launch_q4a).
 __device__ __forceinline__ int any_pad(int k) { return k + (k >> 5) * 4; }
 
 template <bool Q>
@@ -1340,12 +1341,12 @@ hipError_t launch_i4_m1_rows(const Weight& w, size_t m, const float* a, float* o
 }
 
 // Any K and g at M == 1; hipErrorNotSupported where a row's activations and
-// terms exceed 64 KB of LDS.  Rows a workgroup: as many as fit beside the
+// terms exceed 64 KB of LDS (K past about 14000).  Rows a workgroup: as many as fit beside the
 // activations, fewer while the grid is short and a row still fills half the
 // threads.
 hipError_t launch_pack_m1_any(bool q4a, const uint8_t* packed, size_t pitch, const uint16_t* sc, const uint16_t* mn,
                               int ss, size_t n, size_t k, size_t g, const float* a, float* out, hipStream_t s) {
-    if (k == 0 || g == 0 || n > (size_t)INT32_MAX || k > 16384) return hipErrorNotSupported;
+    if (k == 0 || g == 0 || n > (size_t)INT32_MAX || k > 64 * 1024 / 4) return hipErrorNotSupported;
     const size_t gg = std::min(g, k), ng = (k + gg - 1) / gg, row = ((ng + 3) & ~(size_t)3) * 4;
     const size_t act = ((k + k / 32 * 4) / 4 + 4) * 16;
     if (act + row > 64 * 1024) return hipErrorNotSupported;
@@ -1364,9 +1365,11 @@ hipError_t launch_pack_m1_any(bool q4a, const uint8_t* packed, size_t pitch, con
 
 namespace {
 hipError_t i4_m1_any(const Weight& w, const float* a, float* out, hipStream_t s) {
-    const hipError_t e = launch_pack_m1_any(false, w.q4raw, (w.k + 1) / 2, w.s4raw, nullptr, 1, w.n, w.k, w.g, a,
-                                            out, s);
-    if (e != hipErrorNotSupported) return e;
+    if (w.k > 64) {  // a thread a row is the faster below: 37 x 2000 3.5 against 3.9 us, 65 x 2000 5.3 against 4.3
+        const hipError_t e = launch_pack_m1_any(false, w.q4raw, (w.k + 1) / 2, w.s4raw, nullptr, 1, w.n, w.k, w.g, a,
+                                                out, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     i4_gemv_generic<<<dim3((unsigned)((w.n + 255) / 256)), dim3(256), 0, s>>>(w.q4raw, w.s4raw, (int)w.n, (int)w.k,
                                                                              (int)w.g, a, out);
     return hipGetLastError();

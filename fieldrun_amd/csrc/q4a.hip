@@ -164,9 +164,20 @@ hipError_t launch_q4a(const Weight& w, size_t m, const float* a, float* out, hip
             q4a_gemv_kernel<2><<<dim3(grid), dim3(QT), cgb + asb, s>>>(w.q4raw, w.rpitch, w.q4a_sm, (int)w.n,
                                                                       (int)w.k, (int)w.g, rb, a, out);
         else {
-            const uint16_t* sc = reinterpret_cast<const uint16_t*>(w.q4a_sm);
-            const hipError_t e = launch_pack_m1_any(true, w.q4raw, w.rpitch, sc, sc + 1, 2, w.n, w.k, w.g, a, out, s);
-            if (e != hipErrorNotSupported) return e;
+            // groups of 32 or 64 over a ragged K: staged activations and eight
+            // nibbles a load (pack_gemv_any), where the row is long enough to
+            // pay for its staging or the output wide, and several workgroups'
+            // rows fit in a CU's LDS; us here / there: 2310 x 5000 g 32 13.7 /
+            // 12.6, 8001 x 700 14.3 / 9.5, 1001 x 20000 g 64 19.0 / 11.2, but
+            // 790 x 700 4.5 / 4.8, 12001 x 2000 23.5 / 26.8; other groups gain
+            // at some sizes and lose more at others (g 13 4001 x 20000 88 /
+            // 197, g 48 1001 x 2000 3.9 / 4.5, g 128 4001 x 2000 7.5 / 11.0)
+            if ((w.g == 32 || w.g == 64) && w.k <= 8192 && (w.n >= 4096 || w.k >= (w.g == 32 ? 896 : 2048))) {
+                const uint16_t* sc = reinterpret_cast<const uint16_t*>(w.q4a_sm);
+                const hipError_t e = launch_pack_m1_any(true, w.q4raw, w.rpitch, sc, sc + 1, 2, w.n, w.k, w.g, a, out,
+                                                        s);
+                if (e != hipErrorNotSupported) return e;
+            }
             q4a_gemv_kernel<0><<<dim3(grid), dim3(QT), cgb, s>>>(w.q4raw, w.rpitch, w.q4a_sm, (int)w.n, (int)w.k,
                                                                 (int)w.g, rb, a, out);
         }

@@ -111,7 +111,8 @@ def test_expert_banks_in_a_dot_order(ctx, dtype, T, topk, d, mi):
 
 @pytest.mark.parametrize("g", [32, 64, 13, 1, 4000])
 @pytest.mark.parametrize("k,n", [(1, 3), (31, 5), (33, 300), (255, 64), (790, 1), (1001, 700), (6346, 184), (2304, 129),
-                                 (16383, 17), (16400, 9)])
+                                 (16383, 17), (16400, 9), (64, 70), (65, 70), (895, 40), (897, 40), (790, 4096),
+                                 (8191, 20), (8193, 20)])
 def test_one_row_of_any_width_and_group(ctx, k, n, g):
     """M == 1 where the aligned kernels do not apply: the AVX2 orders, groups
     that start inside a byte, rows too long for LDS."""
