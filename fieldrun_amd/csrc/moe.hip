@@ -1339,29 +1339,20 @@ ExpView exp_view(const MoeBank& b, const ExpMat& m) {
     return v;
 }
 
-template <int DT>
-__device__ __forceinline__ float wval(const ExpView& v, size_t e, int k, int j) {
-    if constexpr (DT == FRQ_DT_F32) {
-        return reinterpret_cast<const float*>(v.raw)[e * v.per + (size_t)k * v.out + j];
-    } else if constexpr (DT == FRQ_DT_F16) {
-        return h2f(reinterpret_cast<const uint16_t*>(v.raw)[e * v.per + (size_t)k * v.out + j]);
-    } else {
-        const uint8_t byte = reinterpret_cast<const uint8_t*>(v.raw)[e * v.per + (size_t)j * v.rb + (k >> 1)];
-        const int nib = (k & 1) ? (byte >> 4) : (byte & 15);
-        const size_t gi = e * v.sper + (size_t)j * v.ng + k / v.g;
-        if constexpr (DT == FRQ_DT_I4) return (float)((nib ^ 8) - 8) * h2f(v.sc[gi]);
-        else return h2f(v.sc[gi]) * (float)nib + h2f(v.mn[gi]);
-    }
+// W_e[k, j] of an i4 matrix.
+__device__ __forceinline__ float wval_i4(const ExpView& v, size_t e, int k, int j) {
+    const uint8_t byte = reinterpret_cast<const uint8_t*>(v.raw)[e * v.per + (size_t)j * v.rb + (k >> 1)];
+    const int nib = (k & 1) ? (byte >> 4) : (byte & 15);
+    return (float)((nib ^ 8) - 8) * h2f(v.sc[e * v.sper + (size_t)j * v.ng + k / v.g]);
 }
 
-// x . W_e[:, j] in a.dot's order (MM_KC-long k blocks, each an FMA chain
-// from +0, added in order).
-template <int DT>
-__device__ float exact_ex(const float* __restrict__ x, const ExpView& v, size_t e, int j) {
+// x . W_e[:, j] of an i4 matrix in a.dot's order (MM_KC-long k blocks, each
+// an FMA chain from +0, added in order).
+__device__ float exact_i4(const float* __restrict__ x, const ExpView& v, size_t e, int j) {
     float c = 0.0f;
     for (int k0 = 0; k0 < v.in; k0 += MM_KC) {
         float ab = 0.0f;
-        for (int k = k0; k < min(v.in, k0 + MM_KC); ++k) ab = __builtin_fmaf(x[k], wval<DT>(v, e, k, j), ab);
+        for (int k = k0; k < min(v.in, k0 + MM_KC); ++k) ab = __builtin_fmaf(x[k], wval_i4(v, e, k, j), ab);
         c = c + ab;
     }
     return c;
@@ -1528,7 +1519,7 @@ __device__ __forceinline__ void i4_body(const I4Args& A, uint2 (*As)[I4_AS], con
                 const int j = (cb0 + c) * 16 + col;
                 if (j < A.N) {
                     const float v = so >= 0.0f ? so * acc[t][c]
-                                               : exact_ex<FRQ_DT_I4>(A.xf + (size_t)src * A.K, A.raw, (size_t)e, j);
+                                               : exact_i4(A.xf + (size_t)src * A.K, A.raw, (size_t)e, j);
                     A.y[(size_t)prow * A.N + j] = v;
                 }
             }
@@ -1616,7 +1607,7 @@ __device__ __forceinline__ void i4_body_s(const I4Args& A, uint2* As, const int*
             const int j = (cb0 + c) * 16 + col;
             if (j < A.N) {
                 const float v = so >= 0.0f ? so * (c ? acc1 : acc0)
-                                           : exact_ex<FRQ_DT_I4>(A.xf + (size_t)src * A.K, A.raw, (size_t)e, j);
+                                           : exact_i4(A.xf + (size_t)src * A.K, A.raw, (size_t)e, j);
                 A.y[(size_t)prow * A.N + j] = v;
             }
         }
@@ -1808,8 +1799,8 @@ __global__ __launch_bounds__(256) void moe_i4_dec_gu_kernel(
     i4_dec_loop(qb, sb, dr, kp, ng4, lane, acc);
     const int j = cb * 16 + lane;
     if (lane < 16 && j < mi) {
-        const float gv = ok ? sx * acc[0] : exact_ex<FRQ_DT_I4>(x, G.raw, (size_t)e, j);
-        const float uv = ok ? sx * acc[1] : exact_ex<FRQ_DT_I4>(x, U.raw, (size_t)e, j);
+        const float gv = ok ? sx * acc[0] : exact_i4(x, G.raw, (size_t)e, j);
+        const float uv = ok ? sx * acc[1] : exact_i4(x, U.raw, (size_t)e, j);
         h[(size_t)slot * mi + j] = silu(gv) * uv;
     }
 }
@@ -1858,7 +1849,7 @@ __global__ __launch_bounds__(1024) void moe_i4_dec_dn_kernel(const float* __rest
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int j = (cb0 + c) * 16 + lane;
-            if (j < dn) vs[slot][16 * c + lane] = ok ? so * acc[c] : exact_ex<FRQ_DT_I4>(hr, D.raw, (size_t)e, j);
+            if (j < dn) vs[slot][16 * c + lane] = ok ? so * acc[c] : exact_i4(hr, D.raw, (size_t)e, j);
         }
     }
     __syncthreads();
