@@ -110,12 +110,37 @@ def test_config2_gemma2_2b_int4(ctx, tmp_path):
     b.close()
 
 
-def test_gemma_prefill_ignores_non_finite_values_behind_window(ctx, tmp_path):
+@pytest.mark.parametrize("n_head,n_kv,hd", [(2, 1, 32), (6, 1, 32), (2, 1, 64)])
+def test_gemma_prefill_sliding_window_matches_oracle(ctx, tmp_path, n_head, n_kv, hd):
+    """The two-launch prefill attention (1024 rows and more, head widths of
+    32 and 64, two and eight head slots) with a sliding layer under a global
+    one, the window's lower edge inside the prompt: the oracle's bits."""
+    stem = str(tmp_path / "w")
+    synth.write_gemma2_bundle(stem, 28, n_layer=2, n_head=n_head, n_kv=n_kv, hd=hd, d=64, ffn=64, vocab=300, std=0.1,
+                              norm_std=0.1)
+    m, arrs = oracle.read_bundle(stem)
+    ref = oracle.Gemma(m, arrs, nthreads=16)
+    b = fa.Bundle(stem, ctx)
+    g = fa.Gemma(b)
+    prompt = synth.gpt2_prompt(4230, 300, 6)
+    toks, lg = g.generate(prompt, 2, with_logits=True)
+    rt, rlg = ref.generate(prompt, 2, with_logits=True)
+    assert np.array_equal(toks, rt)
+    assert same_bits(lg, rlg), first_diff(lg, rlg)
+    g.free()
+    b.close()
+
+
+@pytest.mark.parametrize("at_row", [5, 100])
+def test_gemma_prefill_ignores_non_finite_values_behind_window(ctx, tmp_path, at_row):
     """A token whose layer-0 value row is not finite, more than the window
     behind the prompt's last row, takes no part in that row's attention
     (prompts of 1024 rows and more): the same logits as with a finite token
     there.  That token's embedding is 3e38 in one channel: infinite once
-    scaled, NaN after the norm, and a logit that the final cap bounds."""
+    scaled, NaN after the norm, and a logit that the final cap bounds.  Row 5
+    shares its 64-key chunk with no key the last rows see; row 100 shares it
+    with some (the last row's first is 104), which the kernel then adds key by
+    key, so those sums are compared too."""
     stem = str(tmp_path / "n")
     synth.write_gemma2_bundle(stem, 18, n_layer=1, n_head=2, n_kv=1, hd=32, d=64, ffn=64, vocab=300, std=0.1,
                               embed="f32")
@@ -131,7 +156,7 @@ def test_gemma_prefill_ignores_non_finite_values_behind_window(ctx, tmp_path):
     b = fa.Bundle(stem, ctx)
     g = fa.Gemma(b)
     toks, lg = g.generate(prompt, 1, with_logits=True)
-    prompt[5] = bad
+    prompt[at_row] = bad
     tb, lgb = g.generate(prompt, 1, with_logits=True)
     assert np.isfinite(lg).all() and np.array_equal(tb, toks)
     assert same_bits(lgb, lg)
