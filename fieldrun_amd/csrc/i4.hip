@@ -1275,7 +1275,8 @@ hipError_t launch_i4_terms(const Weight& w, const float* a, float* out, hipStrea
 }
 
 // Whether launch_i4_rows_a4 takes this weight (else launch_i4_m1_rows runs
-// the rows one M == 1 launch at a time).
+// the rows one M == 1 launch at a time: other shapes, and matrices of 4 GB and
+// more, at which the batched kernels have not been run).
 bool i4_rows_a4_ok(const Weight& w) {
     return (w.g == 32 || w.g == 64) && w.k > 0 && w.k % w.g == 0 && w.k <= (size_t)INT32_MAX &&
            w.n <= (size_t)INT32_MAX && w.n * w.k / 2 < ((size_t)1 << 32);

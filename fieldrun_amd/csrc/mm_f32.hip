@@ -265,7 +265,8 @@ using Weights = std::conditional_t<
     DT == FRQ_DT_F16 || DT == FRQ_DT_F32, Columns<DT == FRQ_DT_F16 ? FRQ_DT_F16 : FRQ_DT_F32, NT>,
     std::conditional_t<GM == 2, PackedAny<DT, NT>, Packed<DT, NT, GM == 1>>>;
 
-// GR: the rows of one expert's tile (MmGroup), else rows 0 .. M - 1.
+// GR: the rows of one expert's tile (MmGroup), else rows 0 .. M - 1.  Two forms
+// spill a register or two (q4a 1 x 4 over 16 waves, f16 2 x 4 grouped).
 template <int DT, int MT, int NT, int P, int GM, bool GR>
 __global__ __launch_bounds__(64 * (P == 1 ? 4 : P), P == 16 ? 4 : MT * NT >= 8 || GM || P == 8 ? 2 : 3) void mm_f32_kernel(
     MmWeight w, MmGroup grp, const float* __restrict__ a, int M, int tm, int tn, float* __restrict__ out) {

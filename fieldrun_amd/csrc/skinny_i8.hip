@@ -272,7 +272,7 @@ hipError_t launch_mid_i8(const Weight& w, size_t m, const int8_t* a8, const floa
                          const float* oval, float* out, int32_t* acc, hipStream_t s) {
     // a8: m rows of pitch Kp; wblk / wkn padded to Np (a multiple of 256)
     if (m < 1 || m > 65535 || !w.wblk || !w.wkn || w.kp % 64 || w.kp == 0) return hipErrorInvalidValue;
-    // two column blocks a wave from 1500 tiles on (us, one / two: K=896 N=4864
+    // two column blocks a wave from 1500 tiles on (us of the kernel, one / two: K=896 N=4864
     // M=48 11.8 / 11.4, M=129 19.9 / 17.9, M=512 55 / 41; K=4096 N=14336 M=20
     // 31.7 / 21.1; K=2048 N=2048 M=129 12.3 / 15.5, M=256 20.0 / 15.9)
     if ((w.n + 15) / 16 * ((m + 15) / 16) > 1500) return launch_m<2>(w, m, a8, sa, oidx, oval, out, acc, s);
