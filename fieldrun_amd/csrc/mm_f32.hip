@@ -19,10 +19,10 @@
 // in the k loop): activations and packed weights are loaded in whole cache
 // lines under the MFMAs of the chunk before.  What bounds it: the f32 MFMAs
 // share the SIMD's pipe with the VALU, which forms the weights (two
-// instructions a value): 1500 clocks a chunk of 1024 MFMA clocks at MT = 1.
+// to three instructions a value): 1500 clocks a chunk of 1024 MFMA clocks at MT = 1.
 // Measured against the kernels it replaced (a lane a row of the output's
 // columns; DPP-broadcast weights), us: int4 300 x 2304 x 9216 3250 (frq_mm)
-// / 240 -> 150 (41 T FMA/s), 1024 x 2304 x 9216 -> 410 (53), q4a 64 x 9216 x
+// / 240 -> 153 (42 T FMA/s), 1024 x 2304 x 9216 -> 438 (50), q4a 64 x 9216 x
 // 2304 400 -> 83.
 //
 // P == 1: four independent waves a workgroup, each keeping the running block
