@@ -259,10 +259,9 @@ hipError_t launch_m(const Weight& w, size_t m, const int8_t* a8, const float* sa
 // workgroups in a third round (32 x 512 x 40000: 43 against 34 exact).  Timed on
 // both routes at 1800 products of K 32 .. 20480, N 64 .. 65000, M 17 .. 4096:
 // none that this rule picks is slower by more than 7% (K = 384; 3% from 512).
-// The GEMM's limits stay: K to 20480.
+// K beyond 20480, which the GEMM does not hold, is served here alone.
 bool mid_i8_ok(const Weight& w, size_t m) {
-    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64 || w.kp > 20480 || w.n > 32768)
-        return false;
+    if (m <= 16 || m > 65535 || !w.wblk || !w.wkn || w.kp == 0 || w.kp % 64 || w.n > 32768) return false;
     const double tiles = (double)((w.n + 15) / 16) * (double)((m + 15) / 16);
     const double cut = w.kp < 256 ? 13000.0 : w.kp < 512 ? 17000.0 : 30000.0;
     return tiles * (3.2 + 0.0019 * (double)w.kp) <= cut;

@@ -114,17 +114,20 @@ def test_i8_gemm_acc_exact_out_within_tol(ctx, m, k, n):
         assert takes_gemm(out, ref)
 
 
-def test_i8_long_rows_of_prompts_are_refused(ctx):
-    """More than 16 rows of K beyond 20480 are refused at any N (the decode
-    kernels take such rows), and the context stays usable."""
+@pytest.mark.parametrize("m,k,n", [(17, 20481, 64), (40, 24576, 300)])
+def test_i8_long_rows_of_prompts(ctx, m, k, n):
+    """More than 16 rows of K beyond 20480, which the GEMM does not hold, on
+    the one-pass tiles; too many of them for the tiles are refused, and the
+    context stays usable."""
     import fieldrun_amd as fa
-    for m, k, n in ((17, 20481, 64), (40, 24576, 300)):
-        a, wt, scale = case(m, k, n, 900 + m)
-        w = ctx.upload_i8(wt, scale)
-        with pytest.raises(fa.FrqError):
-            w.mm(a)
-        got = w.mm(a[:3])
-        assert np.array_equal(got.view(np.uint32), oracle.mm_i8(a[:3], wt, scale).view(np.uint32))
+    a, wt, scale = case(m, k, n, 900 + m)
+    w = ctx.upload_i8(wt, scale)
+    out, acc, *_ = w.mm_debug(a)
+    ref, racc = oracle.mm_i8(a, wt, scale, with_acc=True)
+    assert np.array_equal(acc, racc) and np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+    with pytest.raises(fa.FrqError):
+        w.mm(np.zeros((4096 * 64 // n, k), np.float32))
+    assert np.array_equal(w.mm(a).view(np.uint32), ref.view(np.uint32))
 
 
 def test_i8_activation_edge_cases(ctx):
