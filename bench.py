@@ -1,8 +1,8 @@
 #!/usr/bin/env python3
 """Benchmark of the quantised-linear hot path on one MI355X.
 
-Headline (BASELINE.json metric "decode tok/s & GEMV HBM GB/s (int8/int4);
-prefill int8 TOPS vs MFMA peak") on configs[4], the largest single-GPU
+Headline (metric "decode tok/s & GEMV HBM GB/s (int8/int4);
+prefill int8 TOPS vs MFMA peak") on the largest single-GPU
 configuration: a Qwen2.5-7B-shaped int8 bundle (28 layers, d 3584, 28 / 4
 heads of 128, ffn 18944, vocab 152064; seeded random int8 linears, per-token
 outlier-aware int8 activations), a 2048-token seeded prompt prefilled, then
@@ -33,10 +33,10 @@ same with the AVX-512BW dot the production x86 build dispatches to.
 `parity`: the timed generate's tokens (and, in an untimed call, every
 logits row's SHA-256) against the oracle's fixture (tests/golden).
 
-`detail` holds the other configs and legs: configs[1]'s isolated int8
+`detail` holds the other workloads and legs: the isolated int8
 sweep (M = 1, 4, 16, 128, 2048), int4 / q4a GEMVs at Gemma-2 shapes, the
-unembed row dot, configs[3]'s MoE layer, configs[0] GPT-2 decode and
-configs[2] Gemma-2-2b int4 decode, each with its oracle check.
+unembed row dot, the Qwen3-MoE layer, GPT-2 decode and
+Gemma-2-2b int4 decode, each with its oracle check.
 """
 import argparse
 import json
@@ -53,7 +53,7 @@ sys.path.insert(0, os.path.join(ROOT, "tests", "golden"))
 METRIC = "decode tok/s & GEMV HBM GB/s (int8/int4); prefill int8 TOPS vs MFMA peak"
 HBM_PEAK_GBS = 8000.0
 INT8_PEAK_TOPS = 5000.0
-# configs[4]
+# the headline: Qwen2.5-7B's shapes
 C4 = dict(L=28, H=28, KV=4, hd=128, d=3584, ffn=18944, vocab=152064, prompt=2048, n_new=128)
 C4_SHAPES = [(3584, 4608), (3584, 3584), (3584, 2 * 18944), (18944, 3584)]  # (K, N) of one layer's linears
 PMC_COPY_BYTES = 256 << 20
@@ -126,7 +126,7 @@ def traffic_from(summary):
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
-    ap.add_argument("--steps", type=int, default=3, help="timed configs[4] generate calls")
+    ap.add_argument("--steps", type=int, default=3, help="timed generate calls of the headline")
     ap.add_argument("--warmup", type=int, default=1)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-detail", action="store_true")
@@ -139,11 +139,11 @@ def main():
                     help="also time hipBLASLt's int8 GEMM (torch._int_mm) at the prefill GEMM shapes, a speed "
                          "reference for roofline_prefill (imports torch: not in the default run)")
     ap.add_argument("--only-gemma2", action="store_true",
-                    help="only configs[2]'s Gemma-2 decode (batch 1 and batch 16) and print its detail entry "
+                    help="only the Gemma-2 decode (batch 1 and batch 16) and print its detail entry "
                          "(for profiling those runs; combine with --no-graphs under rocprofv3)")
     ap.add_argument("--pmc-what", default="layer", choices=["layer", "int4", "m128", "moe", "moe4"],
-                    help="counter workload: the configs[4] layer's four decode linears (default), the int4 "
-                         "M=1 GEMV at the Gemma-2 shapes, the int8 linear at M=128, or configs[3]'s MoE "
+                    help="counter workload: the Qwen2.5-7B layer's four decode linears (default), the int4 "
+                         "M=1 GEMV at the Gemma-2 shapes, the int8 linear at M=128, or the Qwen3-MoE "
                          "layer at T=1 and T=512")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
@@ -172,7 +172,7 @@ def main():
         return e0.elapsed_ms(e1) / iters
 
     def decode_linears():
-        """The configs[4] layer's four linear shapes at M=1 (the engine's
+        """The Qwen2.5-7B layer's four linear shapes at M=1 (the engine's
         kernel), each rotated over n_rot sets: per-launch us and algorithmic
         bytes."""
         rows = []
@@ -219,7 +219,7 @@ def main():
                     w.free()
             return
         if args.pmc_what in ("moe", "moe4"):
-            # configs[3]: the Qwen3-MoE routed layer at T=1 and T=512, 9 calls each (moe4: int4 experts, g 32)
+            # the Qwen3-MoE routed layer at T=1 and T=512, 9 calls each (moe4: int4 experts, g 32)
             E, d, mi, topk = 128, 2048, 768, 8
             if args.pmc_what == "moe":
                 gate, gs, up, us_, down, ds = synth.moe_layer(E, d, mi, synth.seed(3))
@@ -273,7 +273,7 @@ def main():
         print(json.dumps({"gemma2_decode": gemma2_detail(args, ctx, fa, cfx, log)}))
         return
 
-    # ======================= headline: configs[4] =======================
+    # ======================= headline: Qwen2.5-7B =======================
     with tempfile.TemporaryDirectory(dir=shm_dir()) as tmp:
         stem = os.path.join(tmp, "qwen25_7b")
         t0 = time.time()
@@ -450,7 +450,7 @@ def main():
 def vendor_int8_gemm(log=lambda *a: None):
     """hipBLASLt's int8 GEMM through torch._int_mm (A (M,K) i8 row-major, B
     (K,N) the transpose of an (N,K) row-major i8 weight, i32 out) at the
-    configs[4] prefill shapes, weights rotated over >= 4 sets: a speed
+    Qwen2.5-7B prefill shapes, weights rotated over >= 4 sets: a speed
     reference for the MFMA GEMM, not a parity path."""
     import torch
     res = {}
@@ -480,7 +480,7 @@ def vendor_int8_gemm(log=lambda *a: None):
 
 def run_detail(args, ctx, fa, hip, synth, convert, time_loop, log, threads, cfx):
     detail = {}
-    # ---------------- configs[1]: the isolated int8 sweep ----------------
+    # ---------------- the isolated int8 sweep ----------------
     shapes = list(synth.SWEEP_KN)
     weights, acts = [], []
     for si, (k, n) in enumerate(shapes):
@@ -603,7 +603,7 @@ def run_detail(args, ctx, fa, hip, synth, convert, time_loop, log, threads, cfx)
                                           "frac": round(gb / HBM_PEAK_GBS, 3)}
         t.free()
     log(f"rowdot {detail['unembed_rowdot']}")
-    # ---------------- configs[3]: the Qwen3-MoE routed layer ----------------
+    # ---------------- the Qwen3-MoE routed layer ----------------
     detail["moe_qwen3_layer"] = {}
     E, d, mi, topk = 128, 2048, 768, 8
     gate, gs, up, us_, down, ds = synth.moe_layer(E, d, mi, synth.seed(3))
@@ -647,7 +647,7 @@ def run_detail(args, ctx, fa, hip, synth, convert, time_loop, log, threads, cfx)
                                                    "TFLOPs": round(2 * T * topk * 3 * d * mi / (us * 1e-6) / 1e12, 2)}
     bank.free()
     log(f"moe int4 {detail['moe_qwen3_layer_int4']}")
-    # ---------------- configs[0]: GPT-2 small greedy decode ----------------
+    # ---------------- GPT-2 small greedy decode ----------------
     detail["gpt2_decode"] = {}
     with tempfile.TemporaryDirectory(dir=shm_dir()) as tmp:
         stem = os.path.join(tmp, "gpt2")
@@ -672,7 +672,7 @@ def run_detail(args, ctx, fa, hip, synth, convert, time_loop, log, threads, cfx)
                 "decode_tok_s": round(1e3 / dec_ms, 1), "prefill_plus_first_ms": round(runs[1] * 1e3, 3)}
             g.free()
         if not args.no_cpu:
-            import oracle  # configs[0]'s CPU rate: the reference's GPT-2 decode restated in C
+            import oracle  # GPT-2's CPU rate: the reference's GPT-2 decode restated in C
 
             m_, arrs = oracle.read_bundle(stem)
             ref = oracle.Gpt2(m_, arrs, nthreads=threads)
@@ -691,7 +691,7 @@ def run_detail(args, ctx, fa, hip, synth, convert, time_loop, log, threads, cfx)
 
 
 def gemma2_detail(args, ctx, fa, cfx, log):
-    """configs[2]: Gemma-2-2b int4 greedy decode, batch 1 and batch 16."""
+    """Gemma-2-2b int4 greedy decode, batch 1 and batch 16."""
     out = {}
     with tempfile.TemporaryDirectory(dir=shm_dir()) as tmp:
         stem = os.path.join(tmp, "gemma2")

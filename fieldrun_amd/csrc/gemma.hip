@@ -994,7 +994,7 @@ constexpr int PF_PP = PF_AP + 16;  // p's LDS row: 16 pairs of four keys on all 
 typedef float f4v __attribute__((ext_vector_type(4)));
 static_assert(MM_KC % PF_VK == 0, "a value chunk lies in one a.dot block");
 constexpr size_t PF_MIN_ROWS = 1024;  // shorter prompts take the one-launch kernels (more workgroups)
-constexpr size_t PF_MAX_BYTES = (size_t)2 << 30;  // score buffer cap (570 MB at configs[4]'s 2048 + 128)
+constexpr size_t PF_MAX_BYTES = (size_t)2 << 30;  // score buffer cap (570 MB at Qwen2.5-7B's 2048 + 128 tokens)
 __host__ __device__ inline int pf_rows(int rp) { return PF_AP / rp; }
 
 struct PfRow {

@@ -11,7 +11,7 @@ from . import convert
 
 SEED0 = 0xF1E1D000
 
-# configs[1]: the isolated int8 linear sweep
+# the isolated int8 linear sweep
 SWEEP_M = (1, 4, 16, 128, 2048)
 SWEEP_KN = ((896, 4864), (4864, 896), (896, 151936), (4096, 14336), (14336, 4096))
 
@@ -112,7 +112,7 @@ def gpt2_prompt(n: int, vocab: int, s: int) -> np.ndarray:
 
 def write_gpt2_bundle(stem: str, s: int, n_layer: int = 12, n_head: int = 12, d: int = 768,
                       n_pos: int = 1024, vocab: int = 50257, std: float = 0.02) -> dict:
-    """a GPT-2-small-shaped int8 bundle (convert_gpt2,
+    """A GPT-2-small-shaped int8 bundle (convert_gpt2,
     src/convert.rs:505-545 with dtype int8): wte / wpe / ln_f in f16, LN
     gains 1 and biases 0, the four Conv1D linears per layer int8 from
     (in, out) sources with f16 biases.  Weights ~ N(0, std)."""
@@ -139,7 +139,7 @@ def write_gpt2_bundle(stem: str, s: int, n_layer: int = 12, n_head: int = 12, d:
 
 def write_qwen3moe_layer_bundle(stem: str, s: int, n_exp: int = 128, d: int = 2048, mi: int = 768,
                                 topk: int = 8, std: float = 0.02, dtype: str = "int8") -> dict:
-    """one Qwen3-MoE routed layer as convert_qwen3moe writes it
+    """One Qwen3-MoE routed layer as convert_qwen3moe writes it
     (src/convert.rs:872-936, every linear put_lin at the converter's dtype:
     "int8", "int4", "q4a", "f16" or "f32"): the router l0.gate and the
     experts l0.experts.{e}.gate / .up / .down, each from an (out, in) Linear
@@ -186,7 +186,7 @@ def _f16_table_chunks(ss, rows: int, d: int, std: float):
 def write_gemma2_bundle(stem: str, s: int, n_layer: int = 26, n_head: int = 8, n_kv: int = 4, hd: int = 256,
                         d: int = 2304, ffn: int = 9216, vocab: int = 256000, std: float = 0.02,
                         dtype: str = "int4", norm_std: float = 0.0, raw: bool = False, embed: str = "f16") -> dict:
-    """a Gemma-2-2b-shaped bundle as convert_gemma writes it
+    """A Gemma-2-2b-shaped bundle as convert_gemma writes it
     (src/convert.rs:636-657 via write_layers 1266-1300): the f16 embed (tied
     unembed), the RMSNorm gains with the +1 baked in (1 + w, w = 0 at init,
     or N(0, norm_std)), and the seven projections per layer put_lin from
@@ -194,7 +194,7 @@ def write_gemma2_bundle(stem: str, s: int, n_layer: int = 26, n_head: int = 8, n
     config [nl, H, nkv, hd, d, ffn, vocab, tied]; config_f [theta, eps,
     attn_cap, final_cap, query_pre_attn_scalar, sqrt(d)] as Gemma-2-2b.
     raw: the int4 linears as seeded random nibbles with f16 scales written
-    directly (the configs[2] size in seconds rather than minutes).
+    directly (the 2B size in seconds rather than minutes).
     embed: the tied table's type when not raw, "f16", "f32" or "int8"
     (rowi8 with f16 per-row scales, put_embed_i8)."""
     from .bundle import BundleWriter, manifest
@@ -247,7 +247,7 @@ def write_rope_bundle(stem: str, s: int, n_layer: int = 28, n_head: int = 28, n_
                       d: int = 3584, ffn: int = 18944, vocab: int = 152064, std: float = 0.02, dtype: str = "int8",
                       qkv_bias: bool = True, qk_norm: bool = False, tied: bool = False, norm_std: float = 0.0,
                       theta: float = 1e6, eps: float = 1e-6, raw: bool = False) -> dict:
-    """a Llama / Qwen2.5-7B-shaped bundle as convert_rope writes
+    """A Llama / Qwen2.5-7B-shaped bundle as convert_rope writes
     it (src/convert.rs:619-634 via write_layers 1266-1310): f16 embed (and
     lm_head unless tied), in_ln / post_ln RMSNorm weights (1 at init, or
     1 + N(0, norm_std); no +1 bake), q/k/v biases (Qwen2.5) and per-head

@@ -353,7 +353,7 @@ int frq_gemma_generate(frq_ctx* ctx, frq_gemma* g, const int64_t* prompt, size_t
 int frq_gemma_predict(frq_ctx* ctx, frq_gemma* g, const int64_t* ids, size_t n, int64_t* token,
                       float* logits);
 int frq_gemma_set_graphs(frq_gemma* g, int on);
-/* nb sequences at once (configs[2]'s batch 16): prompts (nb, n_prompt),
+/* nb sequences at once (a batch of 16): prompts (nb, n_prompt),
  * each sequence its own Model::generate (src/gemma.rs:403-431; the reference
  * has no batched generate, a batch is nb independent calls): out (nb, n_new)
  * and logits (nb, n_new, vocab), nullable, are what nb calls of

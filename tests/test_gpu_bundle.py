@@ -108,7 +108,7 @@ def test_bundle_upload_errors(ctx, stem):
 
 
 def test_gpt2_config_bundle_on_device(ctx, tmp_path):
-    """configs[0]'s shapes (GPT-2 small, one layer): each Conv1D linear read
+    """GPT-2 small's shapes (one layer): each Conv1D linear read
     from the bundle and run on the device gives the oracle's bits, and the
     tied f16 wte unembed is the reference's rowdot_f32."""
     stem = str(tmp_path / "gpt2")
@@ -128,7 +128,7 @@ def test_gpt2_config_bundle_on_device(ctx, tmp_path):
 
 
 def test_qwen3moe_config_bundle_on_device(ctx, tmp_path):
-    """configs[3]'s expert shapes (Qwen3-30B-A3B: d 2048, moe_inter 768, top
+    """The Qwen3-MoE expert shapes (Qwen3-30B-A3B: d 2048, moe_inter 768, top
     8) with 16 experts: the router is the bundle's int8 l0.gate through mm,
     and the routed layer from the bundle's expert bank matches the oracle
     (the call-site chain of src/qwen3moe.rs:120-158: router mm, softmax,

@@ -4,10 +4,10 @@ make_config_fixtures.py with the C restatement of Gemma::generate /
 Rope::generate on the same seeded bundles and prompts): the greedy tokens,
 and every generated token's f32 logits row bit for bit (its SHA-256).
 
-configs[4]: Qwen2.5-7B-shaped int8, all 28 layers, the 2048-token prompt
+Qwen2.5-7B-shaped int8, all 28 layers, the 2048-token prompt
 (the engine's MFMA prefill with the exact epilogue, grouped prefill
 attention over 2048 rows) and 128 greedy tokens (long-cache decode to 2175
-positions).  configs[2]: Gemma-2-2b-shaped int4, the 64-token prompt and
+positions).  Gemma-2-2b-shaped int4, the 64-token prompt and
 256 greedy tokens, batch 1, and batch 16 (sixteen prompts decoded together,
 each sequence against its own oracle generate)."""
 import os

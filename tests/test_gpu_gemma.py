@@ -3,7 +3,7 @@ src/gemma.rs:242-441) against the oracle's restatement of the same bundle:
 tokens and logits bit for bit, for int4 / int8 / q4a linears, the f32 and
 int8 caches, prompts of 1, 5, 20 rows, the captured-graph decode equal to
 the eager one, the sliding window (a prompt past 4096 positions), and
-configs[2] (Gemma-2-2b, int4) at full size on a short sample."""
+Gemma-2-2b (int4) at full size on a short sample."""
 import json
 
 import numpy as np
@@ -92,7 +92,7 @@ def test_gemma_errors(ctx, small, tmp_path):
 
 
 def test_config2_gemma2_2b_int4(ctx, tmp_path):
-    """configs[2]: Gemma-2-2b shapes (26 layers, d 2304, 8 / 4 heads of 256,
+    """Gemma-2-2b shapes (26 layers, d 2304, 8 / 4 heads of 256,
     ffn 9216, vocab 256000, int4 g=32, f16 embed), a seeded prompt: tokens
     and logits bit for bit on a short sample (the oracle is a CPU restatement)."""
     stem = str(tmp_path / "g2")
@@ -232,7 +232,7 @@ def test_gemma_cache_past_64k_of_scores(ctx, tmp_path):
 
 @pytest.mark.parametrize("kv_int8", [False, True])
 def test_gemma_batch_matches_single_sequences(ctx, small, kv_int8):
-    """configs[2]'s batch decode: each row of a batch is its own
+    """The batch decode: each row of a batch is its own
     Gemma::generate (the reference has no batched generate), so the batch
     gives, bit for bit, the tokens and logits of one call a sequence, and of
     the oracle (int4 rows in i4_dot_avx2's order, q4a / int8 rows as at

@@ -2,8 +2,8 @@
 src/composition.rs:175-341) against the oracle's restatement on the same
 bundle: identical greedy tokens and bit-identical logits, for the f32 and
 the int8 KV cache, prompts of 1 row, 2..16 rows and more (chunked), the
-captured-graph decode equal to the eager one, and configs[0] (GPT-2 small,
-random init) at full size."""
+captured-graph decode equal to the eager one, and GPT-2 small (random
+init) at full size."""
 import numpy as np
 import pytest
 
@@ -121,7 +121,7 @@ def test_gpt2_errors(ctx, lively, tmp_path):
 
 @pytest.mark.parametrize("kv_int8", [False, True])
 def test_config0_gpt2_small_greedy_tokens(ctx, tmp_path_factory, kv_int8):
-    """configs[0]: GPT-2 small int8, random init (std 0.02), 32-token seeded
+    """GPT-2 small int8, random init (std 0.02), 32-token seeded
     prompt, 128 greedy tokens: identical to the oracle, logits bit for bit."""
     stem = bundle(tmp_path_factory, "config0", 1234)
     m, arrs = oracle.read_bundle(stem)

@@ -6,7 +6,7 @@ bit-exact; int8 f32 outputs bit-exact on the GEMV path (same operation
 order as the oracle) and on the MFMA path within
   |gpu - oracle| <= 1e-6 * |scale| * (|sa*acc| + sum_t |av_t * w_t|)
 per element (the outlier correction runs on 24-bit fixed-point MFMA there);
-int4 within 1e-5 of sum |a*w| per element (north_star allows 1e-4).
+int4 within 1e-5 of sum |a*w| per element (1e-4 is allowed).
 """
 import numpy as np
 import pytest
@@ -195,7 +195,7 @@ def test_i8_bundle_upload_matches_transposed(ctx):
 
 @pytest.mark.parametrize("k,n", synth.SWEEP_KN)
 def test_i8_sweep_full_shapes(ctx, k, n):
-    """configs[1] shapes at full size: M=1, 4 and 16 fully against the
+    """The sweep's shapes at full size: M=1, 4 and 16 fully against the
     oracle, M=128 and M=2048 on sampled rows (rows are independent)."""
     a, wt, scale = case(2048, k, n, synth.seed(1))
     w = ctx.upload_i8(wt, scale)

@@ -108,7 +108,7 @@ CASES = [(1, 16, 256, 64, 4, 0), (40, 16, 256, 64, 4, 0), (7, 8, 130, 40, 8, 1),
 @pytest.mark.parametrize("dtype", list(DTYPES))
 @pytest.mark.parametrize("T,E,d,mi,k,act", CASES)
 def test_moe_ex_layer_parity(ctx, dtype, T, E, d, mi, k, act):
-    """configs[3]'s dims (E 128, d 2048, mi 768, top-8) at T = 1 and 512
+    """The Qwen3-MoE layer's dims (E 128, d 2048, mi 768, top-8) at T = 1 and 512
     among the cases.  q4a / f16 / f32 layers bit-exact; int4 within the
     term bound, routing identical in every case."""
     if dtype != "int4" and T == 512:

@@ -4,7 +4,7 @@ same bundle, tokens and logits bit for bit: Qwen2.5-style (q/k/v biases,
 untied lm_head) int8, Qwen3-style (per-head q/k norms, tied) int4, q4a,
 the f32 and int8 caches, prompts of 1, 5 and 20 rows (the int8 prefill in
 bit-exact chunks), the captured-graph decode equal to the eager one; and
-configs[4]'s width (d 3584, 28 / 4 heads of 128, ffn 18944, vocab 152064)
+Qwen2.5-7B's width (d 3584, 28 / 4 heads of 128, ffn 18944, vocab 152064)
 on two layers."""
 import numpy as np
 import pytest
@@ -72,7 +72,7 @@ def test_rope_rejects_other_archs(ctx, tmp_path):
 
 
 def test_config4_width_two_layers(ctx, tmp_path):
-    """configs[4]'s layer width (Qwen2.5-7B: d 3584, 28 / 4 heads of 128,
+    """Qwen2.5-7B's layer width (d 3584, 28 / 4 heads of 128,
     ffn 18944, vocab 152064, int8 with q/k/v biases, untied head) on two
     layers: a 20-token prompt through the chunked bit-exact int8 prefill,
     then decode, bit for bit."""
